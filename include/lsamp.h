@@ -329,9 +329,10 @@ lsamp_status lsamp_context_read_timing(lsamp_context* ctx, double* stats_ms, dou
 /* Kernel arrangement.  AUTO (default) runs the one-pass top-k kernel when
  * `params_host` shows every row is argmax or CBv2 top-k <= LSAMP_TOPK_MAX_K
  * (each slice of a row publishes its best keys; the slice that starts last
- * merges and draws; no co-residency needed), else one kernel whose grid fits
- * on the device at once (the slices of a row hand their results to each
- * other while the logits stay in registers).  FUSED never takes the top-k
+ * merges and draws; no co-residency needed), else one kernel (the slices of
+ * a row hand their results to each other while the logits stay in registers;
+ * its grid fits on the device at once, but for an fp32 batch larger than
+ * that).  FUSED never takes the top-k
  * kernel; SPLIT runs two kernels with no co-residency requirement (the
  * second re-reads each slice from L2).  All give identical results. */
 #define LSAMP_MODE_AUTO 0
@@ -355,8 +356,9 @@ lsamp_status lsamp_context_read_status(lsamp_context* ctx, uint32_t* bits);
 
 /* Launch shape of the context's last lsamp_sample call (diagnostics; no
  * device work): fused with raw log-probabilities (4, lsamp_step), top-k with
- * raw log-probabilities (3, lsamp_step), top-k (2), fused (1) or split (0),
- * slices per row, tokens per slice, rows per round of the fused grid,
+ * raw log-probabilities (3, lsamp_step), top-k (2), fused on a grid that fits
+ * the device at once (1), or more work-groups than that (0: the split kernels,
+ * or the fused kernel's fp32 batches past one round), slices per row, tokens per slice, rows per round of the fused grid,
  * work-groups per kernel launch. */
 typedef struct lsamp_launch_info {
   int32_t fused;

@@ -242,11 +242,16 @@ lsamp_status lsamp::sample_step(const WorkspaceViews& v, const DeviceShape& d, i
   // (the top-k kernel: one work-group per CU is enough, and fewer slices per
   // row mean a shorter merge)
   plan_slices(a->rows, a->vocab, topk ? d.cus : slots, &P.slices, &P.slice_len, &P.nchunks);
-  // (fp32 steps run fused in one round only: the fused kernel's several-rounds
-  // form is not built for the fp32 slab)
+  // An fp32 batch past one round of the grid (the several-rounds form is not
+  // built for the fp32 slab: it would not fit the registers) runs the one-round
+  // kernel over a grid larger than the device: its hand-off assumes no
+  // co-residency, so the dispatcher's own order serves.  128 rows x 151,936
+  // with top-p: 94 us, the split kernels (which read every slice twice) 102.
+  // With raw log-probabilities asked for, such a batch keeps the split kernels.
+  const bool over = a->dtype == LSAMP_DTYPE_F32 && (int64_t)a->rows * P.slices > slots;
   P.fused = !topk && mode != LSAMP_MODE_SPLIT && bpc > 0 && slots >= P.slices &&
-            (a->dtype != LSAMP_DTYPE_F32 || (int64_t)a->rows * P.slices <= slots);
-  P.rows_per_round = P.fused ? slots / P.slices : a->rows;
+            (!over || !(lp && lp->k >= 0));
+  P.rows_per_round = P.fused && !over ? slots / P.slices : a->rows;
   const size_t es = a->dtype == LSAMP_DTYPE_F32 ? 4 : 2;
   P.aligned = aligned16(a->logits) && ((size_t)a->row_stride * es) % 16 == 0;
   P.logits = a->logits;
@@ -307,7 +312,7 @@ lsamp_status lsamp::sample_step(const WorkspaceViews& v, const DeviceShape& d, i
     flp.ids = lp->ids;
     flp.rec = v.rawrec;
   }
-  last->fused = topk ? (lp_fused ? 3 : 2) : (lp_sample ? 4 : P.fused);
+  last->fused = topk ? (lp_fused ? 3 : 2) : (lp_sample ? 4 : (over ? 0 : P.fused));
   last->slices = P.slices;
   last->slice_len = P.slice_len;
   last->rows_per_round = P.rows_per_round;
@@ -964,9 +969,10 @@ lsamp_status lsamp_verify(lsamp_context* ctx, const lsamp_verify_args* a, void* 
   const int32_t bpc = ctx->shape.fused_bpc[a->dtype];
   const int32_t slots = ctx->cus * (bpc > 0 ? bpc : 1);
   plan_slices(P.rows, P.vocab, slots, &P.slices, &P.slice_len, &P.nchunks);
-  P.fused = ctx->mode != LSAMP_MODE_SPLIT && bpc > 0 && slots >= P.slices &&
-            (a->dtype != LSAMP_DTYPE_F32 || (int64_t)P.rows * P.slices <= slots);
-  P.rows_per_round = P.fused ? slots / P.slices : P.rows;
+  // (fp32 rows past one round: as in sample_step)
+  P.fused = ctx->mode != LSAMP_MODE_SPLIT && bpc > 0 && slots >= P.slices;
+  const bool over = a->dtype == LSAMP_DTYPE_F32 && (int64_t)P.rows * P.slices > slots;
+  P.rows_per_round = P.fused && !over ? slots / P.slices : P.rows;
   const size_t es = a->dtype == LSAMP_DTYPE_F32 ? 4 : 2;
   P.aligned = aligned16(a->target_logits) && (!residual || aligned16(a->draft_logits)) &&
               ((size_t)a->vocab * es) % 16 == 0;

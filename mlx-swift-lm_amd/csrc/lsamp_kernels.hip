@@ -2926,8 +2926,9 @@ __device__ __forceinline__ uint32_t run_task(const Workspace& ws, const SamplePl
 }
 
 // ================================================================ kernels
-// ONE: every row fits one round of the grid (no loop over rounds, so nothing
-// is hoisted out of one and spilled before the first load).
+// ONE: a work-group per task (no loop over rounds, so nothing is hoisted out
+// of one and spilled before the first load): every row fits one round of the
+// grid, or (fp32) the grid is larger than the device.
 // LP: raw log-probabilities in the same pass (lsamp_step); `Lk` is read
 // where it is used (the raw record and the finalize), not held throughout.
 template <int DT, bool ONE, bool LP>
@@ -3049,10 +3050,10 @@ int launch_dt(const Workspace& ws, const SamplePlan& P, const FusedLp* lp, hipSt
     const dim3 grid((unsigned)(rounds_rows * P.slices));
     const FusedLp none{-1, nullptr, nullptr, nullptr, nullptr};
     const FusedLp& lk = lp ? *lp : none;
-    // (fp32 steps run fused only when every row fits one round: the
-    // several-rounds instantiation with the fp32 slab does not fit the
-    // registers, so it is not built, and the planner gives such steps the
-    // split kernels)
+    // (fp32 steps have no several-rounds instantiation: with the fp32 slab it
+    // does not fit the registers.  The planner gives a batch past one round a
+    // grid of one work-group per task, which the dispatcher starts in order as
+    // work-groups end)
     if constexpr (DT == LSAMP_DTYPE_F32) {
       if (lp)
         hipLaunchKernelGGL((k_fused<DT, true, true>), grid, dim3(kThreads), 0, st, ws, P, lk);
