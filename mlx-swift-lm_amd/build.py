@@ -39,7 +39,9 @@ DEVICE = [
     "-fhip-fp32-correctly-rounded-divide-sqrt",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
-SOURCES_HIP = ["lsamp_kernels.hip", "lsamp_topk.hip", "lsamp_rank.hip", "lsamp_commit.hip",
+# compiled once per logits dtype (LSAMP_DT = 0, 1, 2), in parallel
+SOURCES_HIP_DT = ["lsamp_kernels.hip"]
+SOURCES_HIP = ["lsamp_topk.hip", "lsamp_rank.hip", "lsamp_commit.hip",
                "lsamp_mask.hip", "lsamp_noalloc.hip", "lsamp_penalize.hip"]
 SOURCES_CPP = ["lsamp_api.cpp"]
 HEADERS = ["lsamp_internal.h", "lsamp_device.h"]
@@ -55,6 +57,12 @@ def build_lib(verbose_asm: bool = False, jobs: int = 0) -> str:
     link liblsamp.so."""
     os.makedirs(LIB_DIR, exist_ok=True)
     cmds, objs = [], []
+    for src in SOURCES_HIP_DT:
+        for dt in range(3):
+            obj = os.path.join(LIB_DIR, src.replace(".hip", f"_{dt}.o"))
+            cmds.append([HIPCC, "-x", "hip", *COMMON, *DEVICE, f"-DLSAMP_DT={dt}", "-c",
+                         os.path.join(CSRC, src), "-o", obj])
+            objs.append(obj)
     for src in SOURCES_HIP:
         obj = os.path.join(LIB_DIR, src.replace(".hip", ".o"))
         cmds.append([HIPCC, "-x", "hip", *COMMON, *DEVICE, "-c", os.path.join(CSRC, src), "-o", obj])

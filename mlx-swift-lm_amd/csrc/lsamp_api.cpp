@@ -50,6 +50,38 @@ lsamp_status lsamp::set_error(lsamp_status st, const char* fmt, ...) {
 
 lsamp_status lsamp::clear_error() { return ok(); }
 
+// The sampling kernels' entry points by dtype (each dtype is compiled apart).
+int lsamp::set_spin_test(int32_t polls) {
+  const int e[3] = {set_spin_test_dt<LSAMP_DTYPE_F32>(polls), set_spin_test_dt<LSAMP_DTYPE_BF16>(polls),
+                    set_spin_test_dt<LSAMP_DTYPE_F16>(polls)};
+  return e[0] ? e[0] : e[1] ? e[1] : e[2];
+}
+
+int lsamp::launch_sample(const Workspace& ws, const SamplePlan& plan, const FusedLp* lp,
+                         void* stream, void* const* events) {
+  switch (plan.dtype) {
+    case LSAMP_DTYPE_F32: return launch_sample_dt<LSAMP_DTYPE_F32>(ws, plan, lp, stream, events);
+    case LSAMP_DTYPE_BF16: return launch_sample_dt<LSAMP_DTYPE_BF16>(ws, plan, lp, stream, events);
+    default: return launch_sample_dt<LSAMP_DTYPE_F16>(ws, plan, lp, stream, events);
+  }
+}
+
+int lsamp::fused_blocks_per_cu(int dtype) {
+  switch (dtype) {
+    case LSAMP_DTYPE_F32: return fused_blocks_dt<LSAMP_DTYPE_F32>();
+    case LSAMP_DTYPE_BF16: return fused_blocks_dt<LSAMP_DTYPE_BF16>();
+    default: return fused_blocks_dt<LSAMP_DTYPE_F16>();
+  }
+}
+
+int lsamp::launch_verify_finish(const Workspace& ws, const VerifyPlan& plan, void* stream) {
+  switch (plan.dtype) {
+    case LSAMP_DTYPE_F32: return launch_verify_finish_dt<LSAMP_DTYPE_F32>(ws, plan, stream);
+    case LSAMP_DTYPE_BF16: return launch_verify_finish_dt<LSAMP_DTYPE_BF16>(ws, plan, stream);
+    default: return launch_verify_finish_dt<LSAMP_DTYPE_F16>(ws, plan, stream);
+  }
+}
+
 namespace {
 
 // Restores the caller's current device on scope exit.
@@ -119,6 +151,15 @@ void plan_slices(int32_t rows, int32_t vocab, int32_t slots, int32_t* slices, in
   *slice_len = cps * kChunk;
   *slices = (nch + cps - 1) / cps;
   *nchunks = nch;
+}
+
+// Rows of top-p / min-p alone go through lists in the one-round kernel.  Where
+// a work-group takes several tasks (16-bit batches past one round) a row's
+// histograms cost about what its lists and their wait do, and a row wider than
+// its lists pays for both: 224 rows x 151,936 (verification) 134 us with
+// histograms alone, 159 with lists; 64 rows in one round 45 and 37.
+int32_t nucleus_lists(int32_t dtype, int64_t tasks, int32_t slots) {
+  return dtype == LSAMP_DTYPE_F32 || tasks <= slots ? kPlanLists : 0;
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -252,6 +293,7 @@ lsamp_status lsamp::sample_step(const WorkspaceViews& v, const DeviceShape& d, i
   P.fused = !topk && mode != LSAMP_MODE_SPLIT && bpc > 0 && slots >= P.slices &&
             (!over || !(lp && lp->k >= 0));
   P.rows_per_round = P.fused && !over ? slots / P.slices : a->rows;
+  P.fused |= nucleus_lists(a->dtype, (int64_t)a->rows * P.slices, slots);
   const size_t es = a->dtype == LSAMP_DTYPE_F32 ? 4 : 2;
   P.aligned = aligned16(a->logits) && ((size_t)a->row_stride * es) % 16 == 0;
   P.logits = a->logits;
@@ -299,7 +341,7 @@ lsamp_status lsamp::sample_step(const WorkspaceViews& v, const DeviceShape& d, i
   // raw log-probabilities in the same launch: the top-k kernel (16-bit
   // logits), or the fused sampling kernel (any dtype)
   const bool lp_fused = topk && lp && lp->k >= 0 && a->dtype != LSAMP_DTYPE_F32;
-  const bool lp_sample = !topk && P.fused && lp && lp->k >= 0;
+  const bool lp_sample = (P.fused & kPlanFused) && lp && lp->k >= 0;
   TopkLp lpk{};
   lpk.k = -1;
   if (lp_fused) lpk = *lp;
@@ -312,12 +354,12 @@ lsamp_status lsamp::sample_step(const WorkspaceViews& v, const DeviceShape& d, i
     flp.ids = lp->ids;
     flp.rec = v.rawrec;
   }
-  last->fused = topk ? (lp_fused ? 3 : 2) : (lp_sample ? 4 : (over ? 0 : P.fused));
+  last->fused = topk ? (lp_fused ? 3 : 2) : (lp_sample ? 4 : (over ? 0 : P.fused & kPlanFused));
   last->slices = P.slices;
   last->slice_len = P.slice_len;
   last->rows_per_round = P.rows_per_round;
   last->grid = topk ? (P.rows + 7) / 8 * 8 * P.slices
-                    : P.fused ? (P.rows < P.rows_per_round ? P.rows : P.rows_per_round) * P.slices
+                    : (P.fused & kPlanFused) ? (P.rows < P.rows_per_round ? P.rows : P.rows_per_round) * P.slices
                               : P.rows * P.slices;
   const int err =
       topk ? launch_topk(P, v.topk, lpk, stream, ev)
@@ -973,6 +1015,7 @@ lsamp_status lsamp_verify(lsamp_context* ctx, const lsamp_verify_args* a, void* 
   P.fused = ctx->mode != LSAMP_MODE_SPLIT && bpc > 0 && slots >= P.slices;
   const bool over = a->dtype == LSAMP_DTYPE_F32 && (int64_t)P.rows * P.slices > slots;
   P.rows_per_round = P.fused && !over ? slots / P.slices : P.rows;
+  P.fused |= nucleus_lists(a->dtype, (int64_t)P.rows * P.slices, slots);
   const size_t es = a->dtype == LSAMP_DTYPE_F32 ? 4 : 2;
   P.aligned = aligned16(a->target_logits) && (!residual || aligned16(a->draft_logits)) &&
               ((size_t)a->vocab * es) % 16 == 0;

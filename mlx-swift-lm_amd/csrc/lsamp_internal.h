@@ -84,6 +84,9 @@ struct SliceSummary {
   double zs;         // short-list rows: sum exp((x - x_max) / T_f) over the slice
   int32_t npub;      // short-list rows: published keys (top-k plus ties)
   float ylo;         // short-list rows: no published key's value is below it
+  // nucleus rows, per wave: its key count (low half) and the value below which
+  // its tokens are not listed; then its part of the slice's sum, in 2^-40
+  uint64_t part[2 * kWaves];
   uint64_t hist[kHist];
 };
 
@@ -298,9 +301,14 @@ constexpr uint32_t kStatusSpinTimeout = 1u;  // a fused-kernel barrier wait time
 // Test hook of the fused kernel's bounded waits (set by lsamp_test_set_spin_limit):
 // 0 = normal; n > 0 = every wait's target is unreachable and it gives up after
 // n polls, so the fail-closed path runs while every kernel still exits.
+template <int DT> int set_spin_test_dt(int32_t polls);
 int set_spin_test(int32_t polls);
 int set_topk_spin_test(int32_t polls);  // the same hook for the top-k kernel's finalizer
 constexpr uint32_t kStatusPenaltyCapacity = 2u;  // a verify position's entries did not fit
+
+// SamplePlan::fused: one kernel (else two), and rows of top-p / min-p alone go
+// through lists (nucleus rows).
+constexpr int32_t kPlanFused = 1, kPlanLists = 2;
 
 // Launch description resolved on the host.
 struct SamplePlan {
@@ -313,7 +321,7 @@ struct SamplePlan {
   int32_t slice_len;       // tokens per slice (multiple of kChunk)
   int32_t nchunks;
   int32_t aligned;         // 16-byte vector loads allowed
-  int32_t fused;           // one co-resident kernel (1) or two kernels (0)
+  int32_t fused;           // kPlanFused, kPlanLists
   int32_t rows_per_round;  // fused: rows processed per round of the grid
   const void* logits;
   const void* logits2;     // rows >= rows_split read logits2 (MTP draft rows)
@@ -398,16 +406,23 @@ struct FusedLp {
 // Work-groups of the top-k kernel that fit on one CU.
 int topk_blocks_per_cu(int dtype);
 
-// Kernel launchers (lsamp_kernels.hip).  Return a hipError_t as int.
+// Kernel launchers (lsamp_kernels.hip, compiled once per dtype).  Return a
+// hipError_t as int.
 // `events` (3 hipEvent_t or NULL) bracket the step: before, between the two
 // kernels (split mode; same as before in fused mode), after.
 // `lp` (or NULL): raw log-probabilities in the same pass (fused steps only).
+template <int DT>
+int launch_sample_dt(const Workspace& ws, const SamplePlan& plan, const FusedLp* lp, void* stream,
+                     void* const* events);
 int launch_sample(const Workspace& ws, const SamplePlan& plan, const FusedLp* lp, void* stream,
                   void* const* events);
 // Work-groups of the fused kernel that fit on one CU (occupancy query).
+template <int DT> int fused_blocks_dt();
 int fused_blocks_per_cu(int dtype);
 // Acceptance, residual / bonus draws and outputs of an MTP verification whose
 // rows were sampled by launch_sample into ws.v* (one work-group per sequence).
+template <int DT>
+int launch_verify_finish_dt(const Workspace& ws, const VerifyPlan& plan, void* stream);
 int launch_verify_finish(const Workspace& ws, const VerifyPlan& plan, void* stream);
 // Exact top-k of raw logits and their log-probabilities (lsamp_rank.hip).
 int launch_rank(const RankPlan& plan, void* stream);

@@ -6,11 +6,16 @@
 //
 //  stats phase   16-byte vector loads of the slice, the grammar mask and the
 //                sparse penalties applied exactly as the reference orders
-//                them, then a histogram of the filter-space logit in 1/32-nat
+//                them, then (rows that lists do not decide) a histogram of the filter-space logit in 1/32-nat
 //                bins (count + fixed-point mass, one packed 64-bit LDS atomic
 //                per token).  The slices' histograms are merged on the
 //                absolute bin grid and the bin holding the top-k / top-p /
 //                min-p cut is located.
+//  lists         rows that a few tokens decide need no histogram: argmax and
+//                top-k rows (short list), and in a one-round grid rows of
+//                top-p / min-p alone (nucleus rows), list their largest tokens
+//                and the row's last arriver draws from the lists.  A row that
+//                its lists cannot decide goes on to the histogram.
 //  select phase  every work-group keeps the tokens above the cut bin (fixed-
 //                point draw weight per 1024-token chunk, and a short list of
 //                them) and lists the tokens inside it.  The last work-group of
@@ -50,13 +55,21 @@ constexpr int kSpinLimit = 1 << 20;                   // ~0.2 s of polling
 __device__ int32_t g_spin_test = 0;
 
 // The fused arrangement's per-row synchronisation words (in the arrive_stats
-// array): arrivals at the exchange in the low half of word 0 and start
-// tickets in its high half (an arrival's atomic returns both counts), claims
+// array): arrivals at the exchanges and start tickets in word 0 (an
+// arrival's atomic returns the counts), claims
 // (bit s: slice s's select; bit kClaimStats + s: its fallback histogram) and
 // departures.  The last slice to leave returns them to zero.  (Split mode
 // counts its arrivals in word 0 alone.)
 constexpr int kSyncArrive = 0, kSyncClaims = 2, kSyncOut = 3;
-constexpr uint32_t kStartOne = 1u << 16, kArriveMask = 0xffffu;
+// Word 0: arrivals at the first exchange of a row of lists in bits 0 - 3, those
+// of nucleus rows whose lists cannot decide the row in bits 4 - 7, arrivals at
+// the histograms' exchange in bits 8 - 11, a nucleus row's verdict (written by
+// the first exchange's last arriver) in bits 12 - 13, start tickets from 16.
+constexpr uint32_t kStartOne = 1u << 16, kWideOne = 1u << 4;
+constexpr int kArriveLists = 0, kArriveHists = 8, kVerdictShift = 12;
+constexpr uint32_t kArriveMask = 0xfu, kWideMask = 0xfu << 4;
+constexpr uint32_t kVerdictDrawn = 1, kVerdictHistogram = 2;
+static_assert(kMaxSlices <= (int)kArriveMask, "a row's arrivals fit their bits");
 constexpr uint32_t kClaimStats = 8;
 static_assert(kMaxSlices <= (int)kClaimStats, "claim bits of both kinds fit one word");
 __device__ __forceinline__ uint32_t* row_sync(const Workspace& ws, int row) {
@@ -71,32 +84,59 @@ __device__ __forceinline__ bool claim_bit(uint32_t* sync, uint32_t bit) {
   return ((old >> bit) & 1u) == 0u;
 }
 
-// Thread 0: the first slice from `from` on, other than `own`, whose claim
-// bit `base + s` this work-group sets (and `from` moves past it); -1 when
-// none is left.
-__device__ __forceinline__ int claim_next(uint32_t* sync, int G, int own, uint32_t base,
-                                          int& from) {
-  for (; from < G; ++from) {
-    if (from == own) continue;
-    if (claim_bit(sync, base + (uint32_t)from)) return from++;
-  }
-  return -1;
+// Thread 0: sets the claim bits `base + s` of every slice s of the row other
+// than `own` in one atomic; returns the slices whose bit this set (bit s).
+// (One by one, the claims cost a round trip a slice, after the finalize of
+// every row on the histogram path.)
+__device__ __forceinline__ uint32_t claim_rest(uint32_t* sync, int G, int own, uint32_t base) {
+  const uint32_t m = ((1u << G) - 1u) & ~(1u << own);
+  const uint32_t old = __hip_atomic_fetch_or(sync + kSyncClaims, m << base, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT);
+  return m & ~(old >> base);
+}
+// Thread 0: the lowest slice of a set, taken out of it; -1 when it is empty.
+__device__ __forceinline__ int next_claimed(uint32_t& set) {
+  if (set == 0u) return -1;
+  const int s = __builtin_ctz(set);
+  set &= set - 1u;
+  return s;
 }
 
-// A bounded wait of the fused kernel (thread 0) for the row's exchange: 1
-// when the arrivals reach `target`; -1 when another work-group set claim bit
+// A bounded wait of the fused kernel (thread 0) for an exchange of the row
+// (kArriveLists or kArriveHists): 1 when the arrivals reach `target`; -1 when another work-group set claim bit
 // `bit` (it does that work itself, so this slice can leave); 0 when the wait
 // gave up (the sticky status bit is raised, and the slice leaves).  Callers
 // wait only when every slice of the row has started, so the arrivals come
 // from work-groups that are running.
 __device__ __forceinline__ int wait_exchange(const Workspace& ws, const uint32_t* sync,
-                                             uint32_t target, uint32_t bit) {
+                                             int which, uint32_t target, uint32_t bit) {
   const int32_t test = __hip_atomic_load(&g_spin_test, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   const uint32_t tgt = test > 0 ? 0xffffffffu : target;
   const int lim = test > 0 ? test : kSpinLimit;
   for (int it = 0;;) {
-    if ((ld_coherent(sync + kSyncArrive) & kArriveMask) >= tgt) return 1;
+    if (((ld_coherent(sync + kSyncArrive) >> which) & kArriveMask) >= tgt) return 1;
     // (claims are rare: every 16th poll looks)
+    if ((it & 15) == 15 && ((ld_coherent(sync + kSyncClaims) >> bit) & 1u)) return -1;
+    if (++it >= lim) {
+      atomicOr(ws.status, kStatusSpinTimeout);
+      return 0;
+    }
+    __builtin_amdgcn_s_sleep(2);
+  }
+}
+
+// The same wait for the outcome of a nucleus row's first exchange: the
+// verdict (kVerdictHistogram as soon as one slice's list cannot decide the
+// row), or -1 / 0 as above.  Every slice of the row has started, and the last
+// of them to arrive writes the verdict without waiting for anyone.
+__device__ __forceinline__ int wait_verdict(const Workspace& ws, const uint32_t* sync,
+                                            uint32_t bit) {
+  const int32_t test = __hip_atomic_load(&g_spin_test, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const int lim = test > 0 ? test : kSpinLimit;
+  for (int it = 0;;) {
+    const uint32_t w = test > 0 ? 0u : ld_coherent(sync + kSyncArrive);
+    if ((w & kWideMask) != 0u) return (int)kVerdictHistogram;
+    if (((w >> kVerdictShift) & 3u) != 0u) return (int)((w >> kVerdictShift) & 3u);
     if ((it & 15) == 15 && ((ld_coherent(sync + kSyncClaims) >> bit) & 1u)) return -1;
     if (++it >= lim) {
       atomicOr(ws.status, kStatusSpinTimeout);
@@ -226,6 +266,11 @@ struct ShortLds {
   uint32_t tcnt[kTauBins];
   uint4 squad[(kQStage + 1) * kThreads];  // slot k of thread t at k * kThreads + t; k = kQStage discards
 };
+// A nucleus row's slice, one wave's maxima and masses (see slice_job).
+struct NucWave {
+  float hi, q_few, q_many, z_few, z_many, n_few, n_many, pad;
+  double z;
+};
 struct TaskLds {
   PhaseLds u;
   ShortLds sh;
@@ -241,6 +286,9 @@ struct TaskLds {
   uint32_t hfl[kMaxSlices];
   int32_t hn[kMaxSlices];
   double hz[kMaxSlices];
+  NucWave nw[kWaves];
+  int32_t mcut[kWaves];  // merge: each wave's first bin at the cut, the count above it
+  int32_t mcnt[kWaves];
   float redf[kWaves];
   float redf2[kWaves];
   int32_t redi[kWaves];
@@ -260,8 +308,10 @@ struct TaskLds {
   int32_t xlast;        // this work-group made the exchange's last arrival
   int32_t job;          // the slice of the claimed job, or -1
   int32_t nraw;         // raw log-probability candidates listed
-  int32_t from_stats;   // claim scans: the next slice to try
-  int32_t from_select;
+  uint32_t stats_left;   // slices claimed and not yet done: their histograms
+  uint32_t select_left;  // and their selects
+  int32_t stats_claimed; // those claims have been made
+  int32_t select_claimed;
   uint32_t flags;
   uint32_t task;  // fused kernel over several rounds: the task taken
 };
@@ -286,7 +336,7 @@ static_assert(kSelQueue >= kThreads / kWaves * 8, "a quad step of a wave fits th
 // total mass, so the scan never needs the bins below the cut.
 // The merge's first round trip, spread over the work-group: every wave reads
 // the slices' top bins and counts, wave 0 the rest of the heads (kept in LDS
-// for merge_wave), and wave s < G the top bins of slice s, which it adds,
+// for merge_bins), and wave s < G the top bins of slice s, which it adds,
 // aligned to the row's top bin, into the merge arrays: 512 bins a slice when
 // the row has more than 4 slices (a batch below them would cost two round
 // trips), else 256 (one).  A cut in those bins needs no further round trip.
@@ -325,7 +375,7 @@ __device__ __forceinline__ void merge_stage(const Workspace& ws, const SamplePla
     L.u.m.mass[i] = 0ull;
   }
   __syncthreads();
-  // the row's top bin over the slices with a finite token (as merge_wave)
+  // the row's top bin over the slices with a finite token (as merge_bins)
   const int32_t rt = wave_max(l < G && hn > 0 ? ht : INT32_MIN);
   const int32_t hn_w = __shfl(hn, wv < G ? wv : 0, 64);
   if (wv < G && hn_w > 0) {
@@ -351,9 +401,10 @@ __device__ __forceinline__ void merge_stage(const Workspace& ws, const SamplePla
 }
 
 template <bool STAGED>
-__device__ __forceinline__ void merge_wave(const Workspace& ws, const SamplePlan& P, int row,
+__device__ __forceinline__ void merge_bins(const Workspace& ws, const SamplePlan& P, int row,
                                            const RowCtx& c, const lsamp_row_params& prm, TaskLds& L) {
-  const int l = fresh_tid();  // lane, wave 0
+  const int tid = fresh_tid();
+  const int l = tid & 63, wv = tid >> 6;
   const int G = P.slices;
   const int64_t V = P.vocab;
   const SliceSummary* summ = ws.summaries + (size_t)row * kMaxSlices;
@@ -390,22 +441,15 @@ __device__ __forceinline__ void merge_wave(const Workspace& ws, const SamplePlan
         w[s][k] = (hist_row && s < G) ? ld_coherent(&summ[s].hist[64 * k + l]) : 0ull;
   }
 
-  float row_max = kNegInf;
-  int32_t row_top = 0, n_total = 0;
+  const bool live = l < G && hn > 0;
+  const bool any = __ballot(live) != 0ull;
+  const float row_max = wave_max(live ? hx : kNegInf);
+  const int32_t row_top = any ? wave_max(live ? htop : INT32_MIN) : 0;
+  const int32_t n_total = wave_sum(live ? hn : 0);
   uint32_t rflags = 0u;
-  bool first = true;
-  for (int s = 0; s < G; ++s) {
-    const float xs = __shfl(hx, s, 64);
-    const int32_t ts = __shfl(htop, s, 64);
-    const int32_t ns = __shfl(hn, s, 64);
-    rflags |= (uint32_t)__shfl((int)hfl, s, 64);
-    n_total += ns;
-    if (ns > 0) {
-      if (first || xs > row_max) row_max = xs;
-      if (first || ts > row_top) row_top = ts;
-      first = false;
-    }
-  }
+#pragma unroll
+  for (uint32_t f : {(uint32_t)LSAMP_ROW_NONFINITE, kSliceEntryOverflow, kSlicePosInf})
+    rflags |= __ballot(l < G && (hfl & f) != 0u) != 0ull ? f : 0u;
   RowInfo info;
   info.x_max = row_max;
   info.top_bin = row_top;
@@ -482,10 +526,62 @@ __device__ __forceinline__ void merge_wave(const Workspace& ws, const SamplePlan
     int cut = -1;
     int32_t cut_c = 0;
     double cut_m = 0.0;
-    for (int b = 0; b < kBins / (64 * kBlk) && cut < 0; ++b) {
+    auto bin_mass = [&](int j, uint32_t cj, uint64_t mj) {
+      return cj ? (double)mj * inv_frac * fexp((double)(row_top - j + 1) * bin_t - q_ref) : 0.0;
+    };
+    auto reached = [&](int j, int32_t C, int32_t cj, double M, double mj) {
+      if (cj == 0 && !(m_on && j == j_t)) return false;
+      const bool tk = k_on && C + cj >= k_lim;
+      const bool tp = p_on && cj > 0 && (strict ? (M + mj >= P_lim) : (M + mj > P_lim));
+      const bool tm = m_on && j >= j_t;
+      return tk || tp || tm;
+    };
+    if constexpr (STAGED) {
+      // the staged bins, one a thread: a wave scans its 64, and the waves'
+      // totals meet in LDS (every wave adds them in the same order)
+      static_assert(kMergeStageBins <= kThreads, "a thread per staged bin");
+      const int nst = 64 * kBlk * staged_batches;
+      const int32_t cj = tid < nst ? (int32_t)L.u.m.cnt[tid] : 0;
+      const double mj = tid < nst ? bin_mass(tid, (uint32_t)cj, L.u.m.mass[tid]) : 0.0;
+      const int32_t ic = wave_incl_scan(cj);
+      const double im = wave_incl_scan(mj);
+      if (l == 63) {
+        L.redi[wv] = ic;
+        L.redd[wv] = im;
+      }
+      __syncthreads();
+      int32_t bc = 0;
+      double bm = 0.0;
+#pragma unroll
+      for (int i = 0; i < kWaves; ++i) {
+        bc += i < wv ? L.redi[i] : 0;
+        bm += i < wv ? L.redd[i] : 0.0;
+        carry_c += L.redi[i];
+        carry_m += L.redd[i];
+      }
+      const int32_t C = bc + ic - cj;
+      const double M = bm + im - mj;
+      const uint64_t hits = __ballot(tid < nst && reached(tid, C, cj, M, mj));
+      if (hits != 0ull && l == __builtin_ctzll(hits)) {
+        L.mcut[wv] = tid;
+        L.mcnt[wv] = C;
+        L.hz[wv] = M;
+      }
+      if (hits == 0ull && l == 0) L.mcut[wv] = -1;
+      __syncthreads();
+      if (wv != 0) return;
+#pragma unroll
+      for (int i = kWaves - 1; i >= 0; --i) {
+        const bool h = L.mcut[i] >= 0;
+        cut = h ? L.mcut[i] : cut;
+        cut_c = h ? L.mcnt[i] : cut_c;
+        cut_m = h ? L.hz[i] : cut_m;
+      }
+    }
+    for (int b = STAGED ? staged_batches : 0; b < kBins / (64 * kBlk) && cut < 0; ++b) {
       uint32_t cnt[kBlk];
       uint64_t msum[kBlk];
-      if (b < staged_batches) {
+      if (!STAGED && b < staged_batches) {
 #pragma unroll
         for (int k = 0; k < kBlk; ++k) {
           cnt[k] = L.u.m.cnt[64 * kBlk * b + 64 * k + l];
@@ -528,20 +624,12 @@ __device__ __forceinline__ void merge_wave(const Workspace& ws, const SamplePlan
         if (cut >= 0) break;
         const int j = 64 * kBlk * b + 64 * k + l;
         const int32_t cj = (int32_t)cnt[k];
-        const double mj = cj ? (double)msum[k] * inv_frac *
-                                   fexp((double)(row_top - j + 1) * bin_t - q_ref)
-                             : 0.0;
+        const double mj = bin_mass(j, (uint32_t)cj, msum[k]);
         const int32_t ic = wave_incl_scan(cj);
         const double im = wave_incl_scan(mj);
         const int32_t C = carry_c + ic - cj;
         const double M = carry_m + im - mj;
-        bool hit = false;
-        if (cj > 0 || (m_on && j == j_t)) {
-          const bool tk = k_on && C + cj >= k_lim;
-          const bool tp = p_on && cj > 0 && (strict ? (M + mj >= P_lim) : (M + mj > P_lim));
-          const bool tm = m_on && j >= j_t;
-          hit = tk || tp || tm;
-        }
+        const bool hit = reached(j, C, cj, M, mj);
         const uint64_t hits = __ballot(hit);
         if (hits) {
           const int f = __builtin_ctzll(hits);
@@ -574,12 +662,12 @@ __device__ __forceinline__ void merge_wave(const Workspace& ws, const SamplePlan
       }
     }
   }
-  if (l == 0) L.info = info;
+  if (tid == 0) L.info = info;
 }
 
 __device__ __forceinline__ void merge_row(const Workspace& ws, const SamplePlan& P, int row, const RowCtx& c,
                           const lsamp_row_params& prm, TaskLds& L) {
-  if (threadIdx.x < 64) merge_wave<false>(ws, P, row, c, prm, L);
+  if (threadIdx.x < 64) merge_bins<false>(ws, P, row, c, prm, L);
   __syncthreads();
 }
 
@@ -620,26 +708,62 @@ struct TailIn {
   int32_t done;     // RowInfo.done of the written row decision
 };
 
-// Keep rule over the sorted candidates, the draw, the probe and the outputs
-// (wave 0 of the finalizing work-group).
-template <int DT>
-__device__ __forceinline__ void finalize_tail(const Workspace& ws, const SamplePlan& P, int row,
-                                              const RowCtx& c, const lsamp_row_params& prm,
-                                              const RowInfo& info, TaskLds& L, const char* rowp,
-                                              const uint32_t* mrow, const TailIn& t,
-                                              uint64_t (&rch)[kChunksPerLane],
-                                              const FusedLp* lp) {
+// A finalized row's outputs and decision (one lane).
+struct RowOut {
+  bool overflow;   // the keep set could not be resolved: fails closed
+  bool draw;       // a token was wanted
+  int32_t token;
+  uint64_t W, probe_w;
+  double ent;      // entropy numerator over the kept
+  float min_kept;
+  int32_t kept, kept_cands, done;
+};
+__device__ __forceinline__ void write_row(const Workspace& ws, const SamplePlan& P, int row,
+                                          const RowInfo& info, float y_max, const RowOut& o) {
+  uint32_t flags = info.flags;
+  if (o.overflow) flags |= LSAMP_ROW_OVERFLOW;
+  if (!o.overflow && ((o.draw && o.token < 0) || o.W == 0ull)) flags |= LSAMP_ROW_EMPTY;
+  const int tok = o.overflow ? -1 : o.token;
+  P.tokens[row] = tok;
+  if (P.row_flags) P.row_flags[row] = flags;
+  if (P.stats) {
+    lsamp_row_stats st;
+    st.max_value = y_max;
+    st.log_normalizer =
+        info.z > 0.0 ? __builtin_logf((float)info.z) + (info.q_top - y_max) : 0.0f;
+    st.kept = o.kept;
+    st.token = tok;
+    st.kept_weight = o.W;
+    st.probe_weight = o.probe_w;
+    st.cut_value = o.min_kept;
+    const double zk = (double)o.W * (1.0 / 1099511627776.0);
+    st.kept_mass = (float)zk;
+    st.kept_entropy = zk > 0.0 ? __builtin_logf((float)zk) - (float)(o.ent / zk) : 0.0f;
+    st.probe_prob = o.W ? (float)((double)o.probe_w / (double)o.W) : 0.0f;
+    P.stats[row] = st;
+  }
+  RowInfo out = info;
+  out.kept_cands = o.overflow ? 0 : o.kept_cands;
+  out.done = o.done;
+  ws.rows[row] = out;
+}
+
+// The keep rule over a row's sorted cut-bin candidates in F.keys (one wave,
+// 64 at a time): the kept ones' weights go to F.rowchunk, F.keep marks them,
+// and they are listed in ws.cands.
+struct KeptCands {
+  int32_t n;
+  double ent;    // entropy numerator
+  float min;     // smallest value
+};
+__device__ __forceinline__ KeptCands keep_candidates(const Workspace& ws, const SamplePlan& P,
+                                                     int row, const RowCtx& c,
+                                                     const lsamp_row_params& prm,
+                                                     const RowInfo& info, FinalLds& F, int nc) {
   const int l = fresh_tid() & 63;
   const int64_t V = P.vocab;
   const float y_max = info.mode == kModePosInf ? kPosInf : to_filter(c, info.x_max);
-  const bool active = info.mode != kModeEmpty;
   Candidate* rc = ws.cands + (size_t)row * kCandCap;
-  FinalLds& F = L.u.f;
-  const int nc = t.nc;
-  const bool overflow = t.overflow;
-  const float u_draw = t.u_draw;
-  const int32_t probe = t.probe;
-  // ---- keep rule over the sorted candidates, 64 at a time
   const double P_lim = info.p_limit;
   const bool p_on = P_lim >= 0.0;
   const int32_t k_lim = (c.kind == LSAMP_KIND_FILTERED && prm.top_k > 0 && (int64_t)prm.top_k < V)
@@ -649,9 +773,6 @@ __device__ __forceinline__ void finalize_tail(const Workspace& ws, const SampleP
   const bool m_on = c.kind == LSAMP_KIND_FILTERED && mp > 0.0f;
   const float ln_mp = m_on ? __builtin_logf(mp) : 0.0f;
   const bool mlx = P.semantics == LSAMP_SEM_MLXLM;
-#pragma unroll
-  for (int i = 0; i < kChunksPerLane; ++i) F.rowchunk[kChunksPerLane * l + i] = rch[i];
-  __builtin_amdgcn_wave_barrier();
   double carry_e = 0.0;
   int32_t carry_s = 0, carry_k = 0;
   double cent = 0.0;
@@ -738,9 +859,39 @@ __device__ __forceinline__ void finalize_tail(const Workspace& ws, const SampleP
     carry_s += read_lane(is, 63);
     carry_k += read_lane(ik, 63);
   }
-  cent = wave_sum(cent);
-  cmin = wave_min(cmin);
-  const int32_t kept_c = carry_k;
+  KeptCands k;
+  k.n = carry_k;
+  k.ent = wave_sum(cent);
+  k.min = wave_min(cmin);
+  return k;
+}
+
+// Keep rule over the sorted candidates, the draw, the probe and the outputs
+// (wave 0 of the finalizing work-group).
+template <int DT>
+__device__ __forceinline__ void finalize_tail(const Workspace& ws, const SamplePlan& P, int row,
+                                              const RowCtx& c, const lsamp_row_params& prm,
+                                              const RowInfo& info, TaskLds& L, const char* rowp,
+                                              const uint32_t* mrow, const TailIn& t,
+                                              uint64_t (&rch)[kChunksPerLane],
+                                              const FusedLp* lp) {
+  const int l = fresh_tid() & 63;
+  const int64_t V = P.vocab;
+  const float y_max = info.mode == kModePosInf ? kPosInf : to_filter(c, info.x_max);
+  const bool active = info.mode != kModeEmpty;
+  FinalLds& F = L.u.f;
+  const int nc = t.nc;
+  const bool overflow = t.overflow;
+  const float u_draw = t.u_draw;
+  const int32_t probe = t.probe;
+  // ---- keep rule over the sorted candidates
+#pragma unroll
+  for (int i = 0; i < kChunksPerLane; ++i) F.rowchunk[kChunksPerLane * l + i] = rch[i];
+  __builtin_amdgcn_wave_barrier();
+  const KeptCands kc0 = keep_candidates(ws, P, row, c, prm, info, F, nc);
+  const double cent = kc0.ent;
+  const float cmin = kc0.min;
+  const int32_t kept_c = kc0.n;
   __builtin_amdgcn_wave_barrier();
 
   // ---- total weight and the chunk holding the target
@@ -931,32 +1082,9 @@ __device__ __forceinline__ void finalize_tail(const Workspace& ws, const SampleP
   }
 
   if (l == 0) {
-    uint32_t flags = info.flags;
-    if (overflow) flags |= LSAMP_ROW_OVERFLOW;
-    if (!overflow && ((draw && token < 0) || W == 0ull)) flags |= LSAMP_ROW_EMPTY;
-    const int tok = overflow ? -1 : token;
-    P.tokens[row] = tok;
-    if (P.row_flags) P.row_flags[row] = flags;
-    if (P.stats) {
-      lsamp_row_stats st;
-      st.max_value = y_max;
-      st.log_normalizer =
-          info.z > 0.0 ? __builtin_logf((float)info.z) + (info.q_top - y_max) : 0.0f;
-      st.kept = t.kept_all + kept_c;
-      st.token = tok;
-      st.kept_weight = W;
-      st.probe_weight = probe_w;
-      st.cut_value = __builtin_fminf(t.min_all, cmin);
-      const double zk = (double)W * (1.0 / 1099511627776.0);
-      st.kept_mass = (float)zk;
-      st.kept_entropy = zk > 0.0 ? __builtin_logf((float)zk) - (float)((t.ent_all + cent) / zk) : 0.0f;
-      st.probe_prob = W ? (float)((double)probe_w / (double)W) : 0.0f;
-      P.stats[row] = st;
-    }
-    RowInfo out = info;
-    out.kept_cands = overflow ? 0 : kept_c;
-    out.done = t.done;
-    ws.rows[row] = out;
+    const RowOut o{overflow, draw, token, W, probe_w, t.ent_all + cent,
+                   __builtin_fminf(t.min_all, cmin), t.kept_all + kept_c, kept_c, t.done};
+    write_row(ws, P, row, info, y_max, o);
     if (t.reset) {
       // (every select of the row has arrived: nothing counts on these any
       // more this step; the exchange's words are cleared by the last slice
@@ -1049,14 +1177,34 @@ __device__ __forceinline__ void finalize_row(const Workspace& ws, const SamplePl
 
   // ---- sort candidates: value descending, id ascending (-0 == +0)
   if (nc > 64 && nc <= kThreads) {
-    // rank by counting (keys are distinct: ids are): one barrier
+    // rank by counting (keys are distinct: ids are), spread over the work-
+    // group: thread (i, ch) counts the keys above key i in chunk ch of the
+    // list (kThreads over nc rounded up to a power of two chunks; 125 keys:
+    // 2.3 us with a thread per key)
+    uint32_t* const above = L.sh.tcnt;
+    static_assert(kTauBins >= kThreads, "a count per candidate");
     if (tid < nc) F.dw[tid] = key0;
+    above[tid] = 0u;
     __syncthreads();
-    if (tid < nc) {
-      int rank = 0;
-      for (int i = 0; i < nc; ++i) rank += F.dw[i] > key0 ? 1 : 0;
-      F.keys[rank] = key0;
+    const int np = nc <= 128 ? 128 : nc <= 256 ? 256 : 512;
+    const int i = tid & (np - 1), span = (nc * np + kThreads - 1) / kThreads;
+    const int j0 = tid / np * span, j1 = j0 + span < nc ? j0 + span : nc;
+    if (i < nc) {
+      const uint64_t key = F.dw[i];
+      int r = 0;
+      int j = j0;
+      for (; j + 8 <= j1; j += 8) {  // (eight reads in flight)
+        uint64_t k8[8];
+#pragma unroll
+        for (int d = 0; d < 8; ++d) k8[d] = F.dw[j + d];
+#pragma unroll
+        for (int d = 0; d < 8; ++d) r = add_gt_u64(r, k8[d], key);
+      }
+      for (; j < j1; ++j) r = add_gt_u64(r, F.dw[j], key);
+      if (r != 0) atomicAdd(&above[i], (uint32_t)r);
     }
+    __syncthreads();
+    if (tid < nc) F.keys[above[tid]] = key0;
     __syncthreads();
   } else if (nc > 64) {
     int n2 = 1;
@@ -2003,6 +2151,626 @@ __device__ __forceinline__ bool short_fallback(const Workspace& ws, int row, int
   return L.misc[5] != 0;
 }
 
+// The first bin of the slice's maxima histogram (L.sh.tcnt, from the top)
+// where the running count reaches `need`; kTauBins when none does.  Whole
+// work-group, the counts complete.
+__device__ __forceinline__ int find_count_bin(TaskLds& L, uint32_t need) {
+  const int tid = fresh_tid();
+            if (tid < 64) {
+              constexpr int kPer = kTauBins / 64;
+              uint32_t cb[kPer];
+              uint32_t cs = 0u;
+  #pragma unroll
+              for (int i = 0; i < kPer; ++i) {
+                cb[i] = L.sh.tcnt[kPer * tid + i];
+                cs += cb[i];
+              }
+              const uint32_t ic = wave_incl_scan(cs);
+              const uint64_t hit = __ballot(ic >= need);
+              int bs = kTauBins;  // the counts never reach `need`
+              if (hit) {
+                // first bin of each lane's run where the running count reaches
+                // k; lane f's is the answer
+                uint32_t acc = ic - cs;
+                int pos = kPer - 1;
+                bool found = false;
+  #pragma unroll
+                for (int i = 0; i < kPer; ++i) {
+                  acc += cb[i];
+                  const bool h = !found && acc >= need;
+                  pos = h ? i : pos;
+                  found = found || h;
+                }
+                const int f = __builtin_ctzll(hit);
+                bs = kPer * f + read_lane(pos, f);
+              }
+              if (tid == 0) L.misc[6] = bs;
+            }
+            __syncthreads();
+  return L.misc[6];
+}
+
+// ============================================================ nucleus rows
+// Rows filtered by top-p and / or min-p alone.  What they keep is usually a
+// few tokens to a few thousand of the row, so a slice does not bin its tokens
+// one by one: it lists its largest ones, and the last arriver takes the
+// lists, bins them, finds the cut and draws, while the other slices are done.
+// (The histogram path spends about 16 VALU operations, an exponential and a
+// 64-bit LDS atomic on every token, exchanges histograms between all slices
+// and goes over the registers again.)
+//
+// A slice lists every token at or above a threshold: the value that a fixed
+// share of its threads' maxima reach (m of 64 maxima at a value mean about
+// -64 ln(1 - m / 64) tokens there), or min-p's own bound when that is higher.
+// The share is small (about 64 tokens a wave) when the maxima that reach it
+// hold top-p of the slice's mass by themselves, else it fills four fifths of
+// the list.  Each wave has its own part of the list, so nothing between the
+// threshold and the published keys waits for another wave.  The lists decide
+// the row when the cut lies above every incomplete part's threshold, which
+// the last arriver checks on the listed masses against the row's total (a sum
+// over every token, from the first pass).  A slice whose list holds less than
+// top-p of its own mass knows that the nucleus is wider than the lists: it
+// sends the row down the histogram path, in the same launch, before the
+// exchange.
+constexpr int kNucP = 1, kNucM = 2;            // a row's filters: top-p, min-p
+constexpr int kNucArea = kCandCap;             // keys of a row in each of two areas:
+static_assert(kMaxSlices * kKeptCap * sizeof(KeptItem) == kNucArea * sizeof(uint64_t),
+              "cands and klist, both idle before the select phase");
+constexpr int kNucPer = 2 * kNucArea / kThreads;  // keys a thread of the last arriver holds
+constexpr int kNucSlices = 4;                  // top-p rows: at most this many slices
+constexpr int kNucFirst = 6;                   // of those, requested with the heads
+constexpr int kNucWaveQuads = (kQStage + 1) * kThreads / kWaves;  // quads a wave stages
+constexpr int kNucWaveKeys = kCandCap / kWaves;                   // keys a wave lists in LDS
+static_assert(offsetof(TaskLds, ssrc) == offsetof(TaskLds, sh) + sizeof(ShortLds) &&
+                  sizeof(ShortLds::squad) + sizeof(TaskLds::ssrc) >=
+                      2 * kNucArea * sizeof(uint64_t),
+              "the last arriver's queues run over both areas");
+static_assert(sizeof(PhaseLds) >= (kHist + 64) * sizeof(uint64_t) +
+                                      kWaves * kNucWaveQuads * sizeof(uint16_t),
+              "the staged quads' numbers fit behind the histogram");
+
+// The filters of a nucleus row (kNucP, kNucM); 0: not one.  Top-p rows of more
+// than four slices (few rows in the batch) are not: a slice's list is half as
+// long there, and one row that its lists cannot decide, which pays for both
+// paths, is the whole step (a row of 151,936 float32 logits that keeps 3,000
+// to 6,600: 41 us on the histogram path, 47 with lists tried first).
+__device__ __forceinline__ int nucleus_filters(const SamplePlan& P, const RowCtx& c,
+                                               const lsamp_row_params& prm) {
+  if (c.kind != LSAMP_KIND_FILTERED || (prm.top_k > 0 && prm.top_k < P.vocab)) return 0;
+  const bool p = top_p_limit(P, c, prm, 1.0) >= 0.0;
+  if (p && P.slices > kNucSlices) return 0;
+  return (p ? kNucP : 0) | (prm.min_p > 0.0f ? kNucM : 0);
+}
+// The two areas hold 8,192 keys: over the slices rounded up to a power of two,
+// and a slice's over its waves (at most 512, what a wave lists in LDS).
+struct NucLayout {
+  int shift;  // log2 of a slice's keys in each area
+  int seg;    // log2 of a wave's keys
+};
+__device__ __forceinline__ NucLayout nucleus_layout(int G) {
+  const int lg = G > 1 ? 32 - __builtin_clz((uint32_t)(G - 1)) : 0;
+  return NucLayout{12 - lg, lg > 0 ? 10 - lg : 9};
+}
+// Key j of slice s of a row.
+__device__ __forceinline__ uint64_t* nucleus_key(const Workspace& ws, int row, int shift, int s,
+                                                 int j) {
+  uint64_t* const a = reinterpret_cast<uint64_t*>(ws.cands + (size_t)row * kCandCap);
+  uint64_t* const b =
+      reinterpret_cast<uint64_t*>(ws.klist + (size_t)row * kMaxSlices * kKeptCap);
+  return ((j >> shift) == 0 ? a + j : b + (j - (1 << shift))) + ((size_t)s << shift);
+}
+
+// Values that at least `m0` and `m1` lanes reach, close to the m-th largest (a
+// bisection between the wave's finite extremes); -inf when fewer are finite.
+__device__ __forceinline__ void wave_reach(float v, float top, int m0, int m1, float& r0,
+                                           float& r1) {
+  const int nf = (int)__popcll(__ballot(v > kNegInf));
+  const float low = wave_min(v > kNegInf ? v : kPosInf);
+  float lo0 = low, hi0 = top, lo1 = low, hi1 = top;
+#pragma unroll 1
+  for (int i = 0; i < 8; ++i) {
+    const float a = lo0 + 0.5f * (hi0 - lo0), b = lo1 + 0.5f * (hi1 - lo1);
+    const bool ka = (int)__popcll(__ballot(v >= a)) >= m0;
+    const bool kb = (int)__popcll(__ballot(v >= b)) >= m1;
+    lo0 = ka ? a : lo0;
+    hi0 = ka ? hi0 : a;
+    lo1 = kb ? b : lo1;
+    hi1 = kb ? hi1 : b;
+  }
+  r0 = nf >= m0 ? lo0 : kNegInf;
+  r1 = nf >= m1 ? lo1 : kNegInf;
+}
+// The share of a wave's 64 thread maxima that its list is sized by: few (which
+// stay within the last arriver's first round trip), or what the list holds.
+__device__ __forceinline__ int nucleus_share(int seg, bool few) {
+  return few ? (seg >= 8 ? 40 : 25) : (seg >= 9 ? 63 : seg == 8 ? 61 : 51);
+}
+
+// This wave's part of a slice's list: the tokens at or above `tau` (and
+// min-p's bound), published as (value bits << 32 | id), with the part's count
+// and threshold and its share `ze` of the slice's mass (see above).  Leaves
+// them in L.hn (-1: it did not fit), L.hx, and the listed mass in L.hz.
+template <int DT, typename F>
+__device__ __forceinline__ void nucleus_list(const Workspace& ws, const SamplePlan& P, int row,
+                                             int slice, const RowCtx& c,
+                                             const lsamp_row_params& prm, int nuc, Slab<DT>& S,
+                                             int nq, int32_t base32, int n_ent, float xmax,
+                                             float tmax, float tau, uint64_t ze, TaskLds& L,
+                                             F&& qmax) {
+  constexpr int N = Vec<DT>::N;
+  const int tid = fresh_tid();
+  const int lane = tid & 63, wv = tid >> 6;
+  const NucLayout lay = nucleus_layout(P.slices);
+  const int cap = 1 << lay.seg;
+  // min-p keeps no token below this (2^-20 covers the roundings of y = x / T,
+  // of y - y_max and of the exponential or logarithm the rule compares)
+  float tm = kNegInf;
+  if (nuc & kNucM) {
+    const float mp = prm.min_p > 1.0f ? 1.0f : prm.min_p;
+    tm = xmax + (float)c.tf * __builtin_logf(mp);
+    tm -= (__builtin_fabsf(xmax) + __builtin_fabsf(tm) + (float)c.tf) * 0x1p-20f;
+  }
+  uint4* const sq = L.sh.squad + wv * kNucWaveQuads;
+  uint16_t* const sid =
+      reinterpret_cast<uint16_t*>(L.u.hist + kHist + 64) + wv * kNucWaveQuads;
+  uint64_t* const lst = L.ssrc + wv * kNucWaveKeys;
+  auto raw = [](float x, int32_t id) {
+    return ((uint64_t)__float_as_uint(x) << 32) | (uint64_t)(uint32_t)id;
+  };
+  auto prefix = [](uint64_t b) {
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32),
+                                          __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0u));
+  };
+  int n = 0;
+  bool fits = false;
+  float tcp = 0.0f;
+  // (a wave whose tokens do not fit tries once more with a few maxima; its
+  // threshold is then higher than the other waves')
+#pragma unroll 1
+  for (int t = 0; t < 2 && !fits; ++t) {
+    if (t > 0) {
+      if (!(nuc & kNucP)) break;
+      float unused;
+      wave_reach(tmax, wave_max(tmax), nucleus_share(lay.seg, true) / 2, 1, tau, unused);
+    }
+    tcp = __builtin_fmaxf(__builtin_fmaxf(tau, tm), -__FLT_MAX__);
+    // the quads that hold a listed token, staged whole
+    int nqd = 0;  // (wave-uniform)
+    for_quads_static(S, nq, [&](int g, uint4& v) -> bool {
+      const bool in = qmax(g, v) >= tcp;
+      const uint64_t b = __ballot(in);
+      if (b != 0ull) {
+        const int o = nqd + prefix(b);
+        if (in && o < kNucWaveQuads) {
+          sq[o] = v;
+          sid[o] = (uint16_t)(g * kThreads + tid);
+        }
+        nqd += (int)__popcll(b);
+      }
+      return false;
+    });
+    fits = nqd <= kNucWaveQuads;
+    if (!fits) continue;
+    __builtin_amdgcn_wave_barrier();
+    // their tokens, a quad a lane, so that every lane works
+    n = 0;
+#pragma unroll 1
+    for (int i0 = 0; i0 < nqd; i0 += 64) {
+      const int i = i0 + lane < nqd ? i0 + lane : 0;
+      const uint4 v = sq[i];
+      const int32_t id0 = base32 + (int32_t)sid[i] * N;
+      const bool live = i0 + lane < nqd;
+#pragma unroll
+      for (int e = 0; e < N; ++e) {
+        const float x = vec_elem<DT>(v, e);
+        const bool in = live && x >= tcp;
+        const uint64_t b = __ballot(in);
+        const int o = n + prefix(b);
+        if (in && o < cap) lst[o] = raw(x, id0 + e);
+        n += (int)__popcll(b);
+      }
+    }
+    // the penalized tokens (their values are in the entry table)
+    for (int j0 = wv * 64; j0 < n_ent; j0 += kThreads) {
+      const int j = j0 + lane;
+      const float x = j < n_ent ? L.ex[j] : kNegInf;
+      const bool in = x >= tcp;
+      const uint64_t b = __ballot(in);
+      const int o = n + prefix(b);
+      if (in && o < cap) lst[o] = raw(x, L.etok[j]);
+      n += (int)__popcll(b);
+    }
+    fits = n <= cap;
+  }
+  float listed = 0.0f;
+  const float lg = (float)(1.4426950408889634 / c.tf);
+  if (fits) {
+    __builtin_amdgcn_wave_barrier();
+    for (int i = lane; i < n; i += 64) {
+      const uint64_t k = lst[i];
+      st_coherent(nucleus_key(ws, row, lay.shift, slice, (wv << lay.seg) + i), k);
+      listed += __builtin_amdgcn_exp2f((__uint_as_float((uint32_t)(k >> 32)) - xmax) * lg);
+    }
+  }
+  listed = wave_sum(listed);
+  const float below = tau <= tm ? kNegInf : tcp;  // (-inf: nothing that could be kept is missing)
+  if (lane == 0) {
+    uint64_t* const head = ws.summaries[(size_t)row * kMaxSlices + slice].part;
+    st_coherent(&head[wv], raw(below, n));
+    st_coherent(&head[kWaves + wv], ze);
+    L.hn[wv] = fits ? n : -1;
+    L.hx[wv] = below;
+    L.hz[wv] = listed;
+  }
+}
+
+// The row from its slices' lists (whole work-group of the last arriver): the
+// listed masses binned, the cut, the tokens above it weighed into chunk sums,
+// those in its bin ranked under the exact keep rule (wave 0), and the draw.
+// False, with the histogram's words zero, when the lists cannot decide the
+// row; the verdict goes to `sync` (fused arrangement, else NULL) as soon as it
+// is known.
+template <int DT>
+__device__ __forceinline__ bool nucleus_row(const Workspace& ws, const SamplePlan& P, int row,
+                                            const RowCtx& c, const lsamp_row_params& prm, int nuc,
+                                            TaskLds& L, const char* rowp, uint32_t* sync,
+                                            const FusedLp* lp) {
+  const int tid = fresh_tid();
+  const int l = tid & 63, wv = tid >> 6;
+  const int G = P.slices;
+  const int64_t V = P.vocab;
+  FinalLds& F = L.u.f;
+  const NucLayout lay = nucleus_layout(G);
+  const SliceSummary* summ = ws.summaries + (size_t)row * kMaxSlices;
+  // one round trip: the heads (in every wave; lane l: wave l % 8 of slice
+  // l / 8) and the first keys of each part (tp threads a part; the keys past
+  // a part's count are dropped once the counts are in)
+  const int tp = kThreads >> (15 - lay.shift);
+  const int part = tid / tp, pos = tid % tp;  // part: slice part / 8, wave part % 8
+  const uint64_t* const kp =
+      nucleus_key(ws, row, lay.shift, part / kWaves, (part % kWaves) << lay.seg) + pos;
+  // (no load is conditional, so that all are in flight together: the areas
+  // exist for every part, and slots past a part's end read its last ones)
+  uint64_t kv[kNucPer];
+#pragma unroll
+  for (int i = 0; i < kNucFirst; ++i) kv[i] = ld_coherent(kp + i * tp);
+  const int hs = l / kWaves, hw = l % kWaves;
+  float hx = kNegInf, hl = kNegInf;
+  int32_t hn = 0, hp = 0;
+  uint32_t hf = 0u;
+  double hz = 0.0;
+  static_assert(kMaxSlices * kWaves == 64, "a lane per wave of the row");
+  if (hs < G) {
+    hx = __uint_as_float(ld_coherent(reinterpret_cast<const uint32_t*>(&summ[hs].x_max)));
+    hn = ld_coherent(&summ[hs].n_finite);
+    hf = ld_coherent(&summ[hs].flags);
+    const uint64_t h = ld_coherent(&summ[hs].part[hw]);
+    hp = (int32_t)(uint32_t)h;
+    hl = __uint_as_float((uint32_t)(h >> 32));
+    hz = (double)ld_coherent(&summ[hs].part[kWaves + hw]) * 0x1p-40;
+  }
+  float u = 0.0f;
+  int32_t pr = -1;
+  if (tid == 0) {
+    if (P.uniforms)
+      u = P.uniforms[uniform_index(P, row)];
+    else if (P.philox_keys)
+      u = philox_uniform(P.philox_keys[row], 0u);
+    const int pi = probe_index(P, row);
+    pr = (P.probe_tokens && pi >= 0) ? P.probe_tokens[pi] : -1;
+    L.misc64[0] = __float_as_uint(u);
+    L.misc64[1] = 0ull;
+    L.misc[4] = pr;
+    L.ncand = 0;
+  }
+  for (int i = tid; i < kBins; i += kThreads) L.u.m.mass[i] = 0ull;
+  for (int i = tid; i < kMaxRowChunks; i += kThreads) F.rowchunk[i] = 0ull;
+  for (int i = tid; i < kChunk + kChunk / 16; i += kThreads) F.dw[i] = 0ull;
+  // (split mode: a slice that cannot be decided from lists says so in its
+  // flags; every wave reads the same ones)
+  if (__ballot((hf & kSliceNoShort) != 0u) != 0ull) return false;
+  const bool live = hs < G && hn > 0;
+  const bool any = __ballot(live) != 0ull;
+  const float row_max = wave_max(live ? hx : kNegInf);
+  const float tstar = wave_max(live ? hl : kNegInf);
+  const bool nonfinite = __ballot(hs < G && (hf & LSAMP_ROW_NONFINITE) != 0u) != 0ull;
+  const int32_t np = live ? hp : 0;
+  const int32_t my_n = __shfl(np, part & 63, 64);
+  // the rest of the longer lists: a second round trip
+  const int slots = (wave_max(np) + tp - 1) / tp;  // (uniform)
+  if (slots > kNucFirst) {
+    const int last = (1 << lay.seg) - tp;
+#pragma unroll
+    for (int i = kNucFirst; i < kNucPer; ++i)
+      kv[i] = ld_coherent(kp + (i * tp < last ? i * tp : last));
+  }
+  const float y_max = any ? to_filter(c, row_max) : 0.0f;
+  const int row_top = any ? bin_of(row_max, c.c32) : 0;
+  // slice s summed exp((x - x_s) / T_f); rescaled to e^y_max
+  const double z = wave_sum(live ? hz * fexp((double)hx / c.tf - (double)y_max) : 0.0);
+  const double P_lim = top_p_limit(P, c, prm, z);
+  __syncthreads();
+  // the listed mass per bin of 1/32 (the histogram path's bins), relative to
+  // e^y_max in 2^40 fixed point; one unit more marks a bin that holds a token
+  constexpr double kLog2e = 1.4426950408889634;
+  const float lg = (float)(kLog2e / c.tf);
+  const float lgl = (float)(kLog2e / c.tf - (double)lg);
+  const float cst = (float)(((double)row_max / c.tf - (double)y_max) * kLog2e);
+#pragma unroll
+  for (int i = 0; i < kNucPer; ++i) {
+    if (i < slots && pos + i * tp < my_n) {
+      const float x = __uint_as_float((uint32_t)(kv[i] >> 32));
+      int b = row_top - bin_of(x, c.c32);
+      b = b < 0 ? 0 : b;
+      if (b < kBins) {
+        const float d = x - row_max;
+        const float e =
+            __builtin_amdgcn_exp2f(__builtin_fmaf(d, lg, __builtin_fmaf(d, lgl, cst)));
+        atomicAdd(reinterpret_cast<unsigned long long*>(&L.u.m.mass[b]),
+                  (unsigned long long)(e * kWeightScale) + 1ull);
+      }
+    }
+  }
+  __syncthreads();
+  // the first bin, from the top, that reaches top-p's limit or min-p's bin
+  // (a thread holds two bins)
+  const bool strict = P.semantics != LSAMP_SEM_CBV2;
+  const bool p_on = P_lim >= 0.0;
+  int32_t j_t = kBins + 1;
+  if (nuc & kNucM) {
+    const float mp = prm.min_p > 1.0f ? 1.0f : prm.min_p;
+    const float st = bin_pos(row_max, c.c32) + (float)(32.0 * c.tf) * __builtin_logf(mp);
+    j_t = row_top - (int32_t)__builtin_floorf(__builtin_fmaxf(st, -1.0e9f));
+    if (j_t < 0) j_t = 0;
+    if (j_t > kBins) j_t = kBins;
+  }
+  const uint64_t m0 = L.u.m.mass[2 * tid], m1 = L.u.m.mass[2 * tid + 1];
+  const uint64_t incl = wave_incl_scan(m0 + m1);
+  if (l == 63) L.redu[wv] = incl;
+  __syncthreads();
+  uint64_t b0 = incl - (m0 + m1);
+#pragma unroll
+  for (int i = 0; i < kWaves; ++i) b0 += i < wv ? L.redu[i] : 0ull;
+  auto hit = [&](int j, uint64_t before, uint64_t mj) {
+    const double after = (double)(before + mj) * 0x1p-40;
+    const bool tp = p_on && mj != 0ull && (strict ? after >= P_lim : after > P_lim);
+    return tp || (j >= j_t && (mj != 0ull || j == j_t));
+  };
+  const bool h0 = hit(2 * tid, b0, m0), h1 = hit(2 * tid + 1, b0 + m0, m1);
+  const uint64_t hm = __ballot(h0 || h1);
+  // (the wave's first hit: its bin and the mass above it)
+  if (hm != 0ull && l == __builtin_ctzll(hm)) {
+    L.redi[wv] = 2 * tid + (h0 ? 0 : 1);
+    L.redd[wv] = (double)(b0 + (h0 ? 0ull : m0)) * 0x1p-40;
+  }
+  if (hm == 0ull && l == 0) L.redi[wv] = 0x7fffffff;
+  __syncthreads();
+  int cut = L.redi[0], at = 0;
+#pragma unroll
+  for (int i = 1; i < kWaves; ++i) {
+    const int ci = L.redi[i];
+    at = ci < cut ? i : at;
+    cut = ci < cut ? ci : cut;
+  }
+  RowInfo info;
+  info.x_max = row_max;
+  info.q_top = y_max;
+  info.top_bin = row_top;
+  info.cut = any ? cut : kCutNone;
+  info.mode = any ? kModeNormal : kModeEmpty;
+  info.flags = nonfinite ? LSAMP_ROW_NONFINITE : 0u;
+  info.count_above = 0;
+  info.n_finite = any ? 1 : 0;
+  info.mass_above = any ? L.redd[at] : 0.0;
+  info.z = z;
+  info.p_limit = P_lim;
+  {
+    int zero = 0, one = 1;  // (made here: see short_gather)
+    asm volatile("" : "+v"(zero), "+v"(one));
+    info.kept_cands = zero;
+    info.done = one;
+  }
+  // decided when every token of the cut bin and above is listed
+  const bool decided = !any || (cut < kBins && cut < row_top - bin_of(tstar, c.c32));
+  if (sync && tid == 0)
+    __hip_atomic_fetch_or(sync + kSyncArrive,
+                          (decided ? kVerdictDrawn : kVerdictHistogram) << kVerdictShift,
+                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (!decided) {
+    for (int i = tid; i < kHist; i += kThreads) L.u.hist[i] = 0ull;
+    return false;
+  }
+  // ---- the kept tokens above the cut bin, and the keys in it
+  const bool active = any;
+  const int32_t probe = L.misc[4];
+  const bool want_stats = P.stats_full != 0;
+  if (P.keep) {
+    uint8_t* kr = P.keep + (size_t)row * (size_t)V;
+    for (int64_t i = tid; i < V; i += kThreads) kr[i] = 0;
+    __syncthreads();
+  }
+  // (the keys of the cut bin and above move to the wave's queue in LDS, so
+  // that the work on them runs with every lane busy)
+  uint64_t* const q = reinterpret_cast<uint64_t*>(L.sh.squad) + wv * (64 * kNucPer);
+  int nq = 0;
+#pragma unroll
+  for (int i = 0; i < kNucPer; ++i) {
+    if (i >= slots) break;
+    const float x = __uint_as_float((uint32_t)(kv[i] >> 32));
+    const bool in = pos + i * tp < my_n && row_top - bin_of(x, c.c32) <= info.cut;
+    const uint64_t b = __ballot(in);
+    if (in)
+      q[nq + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32),
+                                            __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0u))] = kv[i];
+    nq += (int)__popcll(b);
+  }
+  __builtin_amdgcn_wave_barrier();
+  double ent = 0.0;
+  float min_kept = kPosInf;
+  int32_t n_kept = 0;
+#pragma unroll 1
+  for (int i = l; i < nq; i += 64) {
+    const uint64_t k = q[i];
+    const float x = __uint_as_float((uint32_t)(k >> 32));
+    const int32_t id = (int32_t)(uint32_t)k;
+    int j = row_top - bin_of(x, c.c32);
+    j = j < 0 ? 0 : j;
+    const float y = to_filter(c, x);
+    if (j == info.cut) {
+      const int o = atomicAdd(&L.ncand, 1);
+      if (o < kCandCap) F.keys[o] = cand_key(y, id);
+      continue;
+    }
+    const uint64_t w = weight(y, y_max, c.scale);
+    atomicAdd(reinterpret_cast<unsigned long long*>(&F.rowchunk[id / kChunk]),
+              (unsigned long long)w);
+    if (id == probe) L.misc64[1] = w;
+    if (P.keep) P.keep[(size_t)row * (size_t)V + id] = 1;
+    if (want_stats) {
+      ent += (double)w * (1.0 / 1099511627776.0) * (double)weight_arg(y, y_max, c.scale);
+      min_kept = __builtin_fminf(min_kept, y);
+      ++n_kept;
+    }
+  }
+  if (want_stats) {
+    ent = wave_sum(ent);
+    min_kept = wave_min(min_kept);
+    n_kept = wave_sum(n_kept);
+    if (l == 0) {
+      L.hz[wv] = ent;
+      L.hx[wv] = min_kept;
+      L.hn[wv] = n_kept;
+    }
+  }
+  __syncthreads();
+  const bool overflow = L.ncand > kCandCap;
+  const int nc = overflow || !active ? 0 : L.ncand;
+  // the cut bin's keys ranked by counting (keys are distinct: ids are)
+  if (nc > 1) {
+    constexpr int kPer = kCandCap / kThreads;
+    uint64_t key[kPer];
+    int r[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int i = tid + k * kThreads;
+      key[k] = i < nc ? F.keys[i] : 0ull;
+      r[k] = 0;
+      if (k * kThreads < nc && i < nc)
+        for (int j = 0; j < nc; ++j) r[k] = add_gt_u64(r[k], F.keys[j], key[k]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kPer; ++k)
+      if (tid + k * kThreads < nc) F.keys[r[k]] = key[k];
+    __syncthreads();
+  }
+  const bool draw = !P.bonus_only || (row < P.rows_split && row % P.vwin == P.vwin - 1);
+  KeptCands kc{0, 0.0, kPosInf};
+  uint64_t W = 0ull;
+  if (wv == 0) {
+    kc = keep_candidates(ws, P, row, c, prm, info, F, nc);
+    __builtin_amdgcn_wave_barrier();
+    // total weight and the chunk holding the target
+    uint64_t rch[kChunksPerLane];
+    uint64_t lane_w = 0ull;
+#pragma unroll
+    for (int i = 0; i < kChunksPerLane; ++i) {
+      rch[i] = F.rowchunk[kChunksPerLane * l + i];
+      lane_w += rch[i];
+    }
+    const uint64_t iw = wave_incl_scan(lane_w);
+    W = read_lane(iw, 63);
+    const uint64_t target =
+        W ? scaled_target(uniform_u32(__uint_as_float((uint32_t)L.misc64[0])), W) : 0ull;
+    int my_c = -1;
+    uint64_t my_t = 0ull, pre = iw - lane_w;
+#pragma unroll
+    for (int i = 0; i < kChunksPerLane; ++i) {
+      if (rch[i] && pre <= target && target < pre + rch[i]) {
+        my_c = kChunksPerLane * l + i;
+        my_t = target - pre;
+      }
+      pre += rch[i];
+    }
+    const uint64_t hitc = __ballot(my_c >= 0);
+    const bool ok = W && hitc && !overflow && active && draw;
+    if (l == (ok ? __builtin_ctzll(hitc) : 0)) {
+      L.misc[0] = ok ? my_c : -1;
+      L.misc64[2] = my_t;
+    }
+  }
+  __syncthreads();
+  const int cstar = L.misc[0];
+  if (cstar >= 0) {
+    // the chunk's kept tokens to their draw slots
+    for (int i = l; i < nq; i += 64) {
+      const uint64_t k = q[i];
+      const int32_t id = (int32_t)(uint32_t)k;
+      if (id / kChunk != cstar) continue;
+      const float x = __uint_as_float((uint32_t)(k >> 32));
+      if (row_top - bin_of(x, c.c32) < info.cut)
+        F.dw[draw_slot(id % kChunk)] = weight(to_filter(c, x), y_max, c.scale);
+    }
+    for (int r = tid; r < nc; r += kThreads) {
+      const int32_t id = key_id(F.keys[r]);
+      if (F.keep[r] && id / kChunk == cstar)
+        F.dw[draw_slot(id % kChunk)] = weight(key_y(F.keys[r]), y_max, c.scale);
+    }
+  }
+  __syncthreads();
+  if (wv != 0) {
+    // (wave 1: the raw log-probability lists, beside wave 0's draw)
+    if (lp && wv == 1) raw_lists<DT>(P, *lp, row, reinterpret_cast<uint64_t*>(L.sh.squad));
+    return true;
+  }
+  int token = -1;
+  if (cstar >= 0) {
+    const uint64_t ltarget = L.misc64[2];
+    uint64_t sw[kSlotsPerLane];
+    uint64_t lane_s = 0ull;
+#pragma unroll
+    for (int i = 0; i < kSlotsPerLane; ++i) {
+      sw[i] = F.dw[draw_slot(kSlotsPerLane * l + i)];
+      lane_s += sw[i];
+    }
+    uint64_t pre = wave_incl_scan(lane_s) - lane_s;
+    int my_tok = -1;
+#pragma unroll
+    for (int i = 0; i < kSlotsPerLane; ++i) {
+      if (sw[i] && pre <= ltarget && ltarget < pre + sw[i])
+        my_tok = cstar * kChunk + kSlotsPerLane * l + i;
+      pre += sw[i];
+    }
+    const uint64_t hitt = __ballot(my_tok >= 0);
+    if (hitt) token = read_lane(my_tok, __builtin_ctzll(hitt));
+  }
+  uint64_t probe_w = L.misc64[1];
+  if (probe >= 0) {
+    uint64_t pw = 0ull;
+    for (int r = l; r < nc; r += 64)
+      if (F.keep[r] && key_id(F.keys[r]) == probe) pw = weight(key_y(F.keys[r]), y_max, c.scale);
+    const uint64_t hp = __ballot(pw != 0ull);
+    if (hp) probe_w = read_lane(pw, __builtin_ctzll(hp));
+  }
+  if (l == 0) {
+    if (want_stats) {
+      ent = 0.0;
+      min_kept = kPosInf;
+      n_kept = 0;
+      for (int i = 0; i < kWaves; ++i) {
+        ent += L.hz[i];
+        min_kept = __builtin_fminf(min_kept, L.hx[i]);
+        n_kept += L.hn[i];
+      }
+    }
+    const RowOut o{overflow, draw, token, W, overflow ? 0ull : probe_w, ent + kc.ent,
+                   __builtin_fminf(min_kept, kc.min), n_kept + kc.n, kc.n, 1};
+    write_row(ws, P, row, info, y_max, o);
+  }
+  if (lp) raw_chosen<DT>(P, *lp, row, overflow ? -1 : token, rowp);
+  return true;
+}
+
 // What a fused work-group does next on its row (slice_job's result): leave
 // it, or a job for another slice: its fallback histogram (kBehalfStats) or
 // its select (kSelectOnly), from a re-read of that slice.
@@ -2016,7 +2784,7 @@ __device__ __forceinline__ int next_job(int kind, int slice) { return (kind << 8
 // `slice` of a slice that left (kBehalfStats, kSelectOnly); `own` is its own
 // slice.  (Each job is its own instantiation, so the own pass compiles as
 // if the others did not exist.)
-template <int DT, int MODE, int JM, bool LP>
+template <int DT, int MODE, int JM, bool LP, bool NUC>
 __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& P, int row, int slice,
                                          TaskLds& L, int own, const FusedLp& Lk) {
   constexpr int jm = JM;
@@ -2127,12 +2895,17 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
   // integer anchored at a quad maximum (re-anchored by an exact power of two
   // only if the running maximum climbs 64 binary orders above it), so the
   // largest terms are computed at full precision.
-  // (a claimed fallback histogram skips the short list: K = 0; Krow is the
-  // row's own, which sets the exchange's arrival count)
-  const int Krow = jm != kSelectOnly ? short_k(c, prm, V) : 0;
-  const int K = jm == kBehalfStats ? 0 : Krow;
-  const bool zon = K > 0 && c.kind != LSAMP_KIND_ARGMAX;
+  // (a claimed fallback histogram or select skips the row's lists)
+  constexpr bool kOwnLists = jm != kSelectOnly && jm != kBehalfStats;
+  const int K = kOwnLists ? short_k(c, prm, V) : 0;
+  // (split mode lists the rows that the fused kernel would list)
+  const int nuc = kOwnLists && NUC && (MODE == kFused || (P.fused & kPlanLists) != 0)
+                      ? nucleus_filters(P, c, prm)
+                      : 0;
+  const bool zon = (K > 0 && c.kind != LSAMP_KIND_ARGMAX) || (nuc & kNucP) != 0 ||
+                   (nuc != 0 && P.stats != nullptr);
   const float lgz = (float)(1.4426950408889634 / c.tf);  // log2(e) / T_f
+  const float lgl = (float)(1.4426950408889634 / c.tf - (double)lgz);  // its low part
   // penalty-bitmap word of quad g (the bitmap is zeroed over the largest
   // slice, so every quad's word is in bounds); fetched one quad ahead so the
   // LDS read overlaps the current quad
@@ -2210,8 +2983,64 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
     // ------------------------------------------------ B: max
     if (nonfinite) atomicOr(&L.flags, LSAMP_ROW_NONFINITE);
     const float tmax = xmax;  // this thread's largest (transformed) logit
+    const float xthr = tmax;
     float tlo = kPosInf;      // smallest finite thread maximum (short lists, k > 1)
-    if (K > 1) {
+    // nucleus rows: the quads' maxima (16-bit types: kept in the area that the
+    // list overwrites, so read into registers ahead of the barrier)
+    float qv[kKeepQm ? Q : 1];
+    auto qmax = [&](int g, const uint4& v) -> float {
+      if constexpr (kKeepQm) return qv[g];
+      else return vec_max_nn<DT>(v);
+    };
+    if (__builtin_expect(nuc != 0, 0)) {
+      if constexpr (kKeepQm) {
+#pragma unroll
+        for (int g = 0; g < Q; ++g) qv[g] = g < nq ? qmc[g * kThreads + tid] : kNegInf;
+      }
+      // Per wave: its maximum, the values its few and its many maxima reach,
+      // its mass relative to e^(hi / T_f), and the mass and number of the
+      // threads with no token at those values: what such threads hold tells
+      // how much mass lies below them in the whole slice.
+      const int seg = nucleus_layout(G).seg;
+      const float hi = wave_max(tmax);
+      float q_few = kNegInf, q_many = kNegInf;
+      double zsum = 0.0;
+      float z_few = 0.0f, z_many = 0.0f;
+      int n_few = 0, n_many = 0;
+      if (zon && hi > kNegInf && hi < kPosInf) {
+        // (rescaled from 2^-nbz: hi * lgz split into a rounded part and its
+        // exact residual; the low part of log2(e) / T_f taken at the thread's
+        // maximum, near which its mass is)
+        const float bh = hi * lgz;
+        const float bl = __builtin_fmaf(hi, lgz, -bh);
+        const float dl = tmax > kNegInf ? (tmax - hi) * lgl : 0.0f;
+        const float zr = zref ? zt * __builtin_amdgcn_exp2f(((-nbz - bh) - bl) + dl) : 0.0f;
+        zsum = wave_sum((double)zr);
+        if ((nuc & kNucP) != 0) {
+          wave_reach(tmax, hi, nucleus_share(seg, true), nucleus_share(seg, false), q_few, q_many);
+          const bool bf = tmax < q_few, bm = tmax < q_many;
+          z_few = wave_sum(bf ? zr : 0.0f);
+          z_many = wave_sum(bm ? zr : 0.0f);
+          n_few = (int)__popcll(__ballot(bf));
+          n_many = (int)__popcll(__ballot(bm));
+        }
+      }
+      if ((tid & 63) == 0) {
+        NucWave& w = L.nw[tid >> 6];
+        w.hi = hi;
+        w.q_few = q_few;
+        w.q_many = q_many;
+        w.z_few = z_few;
+        w.z_many = z_many;
+        w.n_few = (float)n_few;
+        w.n_many = (float)n_many;
+        w.z = zsum;
+      }
+      __syncthreads();
+      xmax = L.nw[0].hi;
+#pragma unroll
+      for (int i = 1; i < kWaves; ++i) xmax = __builtin_fmaxf(xmax, L.nw[i].hi);
+    } else if (K > 1) {
       float hi = wave_max(tmax);
       float lo = wave_min(tmax > kNegInf ? tmax : kPosInf);
       const int wv = tid >> 6;
@@ -2257,6 +3086,144 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
       for (int j = tid; j < n_ent; j += kThreads) out[L.etok[j]] = to_filter(c, L.ex[j]);
     }
 
+    bool wide = false;  // a nucleus row that its lists cannot decide
+    uint32_t n_word = 0u, n_claim = 0u;  // (then, thread 0) its arrival's and claim's results
+    // (laid out after the other paths, which fall through)
+    if (__builtin_expect(nuc != 0, 0)) {
+      // -------------------------------------------- B': the nucleus list
+      uint32_t* const sync = row_sync(ws, row);
+      const int wv = tid >> 6;
+      // (no list: +inf logits, an entry-table overflow, a sum out of range)
+      const bool bad = posinf || ent_overflow || (zon && has_finite && !(xmax * lgz < 0x1p20f));
+      if (tid == 0) {
+        st_coherent_f32(&Ssum->x_max, xmax);
+        st_coherent(&Ssum->top_bin, top);
+        st_coherent(&Ssum->flags, sflags);
+        st_coherent(&Ssum->n_finite, (has_finite || posinf) ? 1 : 0);
+      }
+      if (has_finite && !bad) {
+        // this wave's part of the slice's sum, relative to e^(xmax / T_f) in
+        // 2^40 fixed point (exact in any order: the entry table's order
+        // depends on atomics); lane i < 8: wave i
+        const NucWave nw = L.nw[tid & 7];
+        const float f = nw.hi > kNegInf ? __builtin_amdgcn_exp2f(__builtin_fmaf(
+                                              nw.hi - xmax, lgz, (nw.hi - xmax) * lgl))
+                                        : 0.0f;
+        const double mass = nw.z * (double)f;
+        uint64_t ze = 0ull;
+        if (zon) {
+          const float nb = -xmax * lgz;
+          const float nb_err = __builtin_fmaf(-xmax, lgz, -nb);
+          const float enb = __builtin_amdgcn_exp2f(nb_err);
+          for (int j = tid; j < n_ent; j += kThreads) {
+            const float x = L.ex[j];
+            if (!(x > kNegInf)) continue;
+            const float a = __builtin_fmaf(x - xmax, lgl, __builtin_fmaf(x, lgz, nb));
+            ze += (uint64_t)(__builtin_amdgcn_exp2f(a) * enb * 0x1p40f);
+          }
+          ze = wave_sum(ze) + (uint64_t)(read_lane(mass, wv) * 0x1p40);
+          if ((tid & 63) == 0) L.redu[wv] = ze;
+        }
+        // The list's size (entries apart): few when the mass below their
+        // threshold is well below what top-p drops, else many, unless even
+        // theirs leaves out more than top-p drops.  The thresholds are the
+        // waves' averaged (a wave with too few finite maxima lists all it has).
+        float tau = kNegInf;
+        if ((nuc & kNucP) != 0) {
+          // (over 8 lanes: two quad permutes and a half-row mirror)
+          auto sum8 = [](float v) {
+            v += dpp_move<0xb1, 0xf>(v, 0.0f);
+            v += dpp_move<0x4e, 0xf>(v, 0.0f);
+            v += dpp_move<0x141, 0xf>(v, 0.0f);
+            return v;
+          };
+          const float all = sum8((float)mass);
+          const float drop = (1.0f - (prm.top_p > 0.0f ? prm.top_p : 0.0f)) * all;
+          const float u_few = sum8(nw.z_few * f) * (float)kThreads;
+          const float u_many = sum8(nw.z_many * f) * (float)kThreads;
+          const float s_few = sum8(nw.n_few), s_many = sum8(nw.n_many);
+          const bool is_few = u_few <= 0.7f * drop * s_few;
+          wide = !is_few && u_many > 0.85f * drop * s_many;
+          const float qw = is_few ? nw.q_few : nw.q_many;
+          const float sum = sum8(qw > kNegInf ? qw : 0.0f);
+          const float cnt = sum8(qw > kNegInf ? 1.0f : 0.0f);
+          if (read_lane(qw, wv) > kNegInf)
+            tau = __uint_as_float(
+                (uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(sum / cnt)));
+        }
+        wide = __builtin_amdgcn_readfirstlane(wide ? 1 : 0) != 0;
+        if (!wide)
+          nucleus_list<DT>(ws, P, row, slice, c, prm, nuc, S, nq, base32, n_ent, xmax, xthr, tau,
+                           ze, L, qmax);
+      } else if (!bad && (tid & 63) == 0) {
+        // (nothing finite)
+        st_coherent(&Ssum->part[wv], (uint64_t)0xff800000u << 32);
+        st_coherent(&Ssum->part[kWaves + wv], (uint64_t)0);
+        L.hn[wv] = 0;
+        L.hx[wv] = kNegInf;
+        L.hz[wv] = 0.0;
+        L.redu[wv] = 0ull;
+      }
+      wide = wide || bad;
+      if (!wide) {
+        drain_memory();
+        __syncthreads();
+        // a part did not fit, or the parts hold less than top-p of the mass
+        double listed = 0.0, mass = 0.0;
+        bool open = false;  // some part is incomplete
+#pragma unroll
+        for (int i = 0; i < kWaves; ++i) {
+          wide = wide || L.hn[i] < 0;
+          open = open || L.hx[i] > kNegInf;
+          listed += L.hz[i];
+          mass += (double)L.redu[i] * 0x1p-40;
+        }
+        wide = wide || ((nuc & kNucP) != 0 && open && listed < (double)prm.top_p * mass);
+      }
+      if (wide) sflags |= kSliceShortOverflow;
+      if (MODE == kFused) {
+        // First exchange of a nucleus row: the last slice to arrive draws
+        // from the lists, or finds that they do not decide the row.  The
+        // others wait for its verdict (as a short-list row's wait for the
+        // arrivals) and go on to the histogram path in the second case.  A
+        // slice that knows it goes on at once: what its arrival and the claim
+        // of its histogram return is looked at when that is built.
+        uint32_t word = 0u, claim = 0u;
+        if (tid == 0) {
+          asm volatile("" ::"v"(tick));
+          word = __hip_atomic_fetch_add(sync + kSyncArrive, wide ? 1u + kWideOne : 1u,
+                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          if (wide)
+            claim = __hip_atomic_fetch_or(sync + kSyncClaims, 1u << (kClaimStats + slice),
+                                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (wide) {
+          n_word = word;
+          n_claim = claim;
+        } else {
+          if (tid == 0) {
+            const bool last = (word & kArriveMask) + 1u == (uint32_t)G;
+            int w = (word & kWideMask) != 0u ? (int)kVerdictHistogram : 0;
+            if (w == 0 && !last && (word >> 16) >= (uint32_t)G)
+              w = wait_verdict(ws, sync, kClaimStats + (uint32_t)slice);
+            L.wait = w;
+            L.last = last ? 1 : 0;
+          }
+          __syncthreads();
+          if (L.last) {
+            if (L.wait == 0 && nucleus_row<DT>(ws, P, row, c, prm, nuc, L, rowp, sync, lpp))
+              return kJobLeave;
+            if (tid == 0) L.x1 = 1;
+          } else if (L.wait != (int)kVerdictHistogram) {
+            return kJobLeave;
+          }
+          // (unless the last arriver has claimed this histogram)
+          if (tid == 0) L.won = claim_bit(sync, kClaimStats + (uint32_t)slice) ? 1 : 0;
+          __syncthreads();
+          if (!L.won) return kJobLeave;
+        }
+      }
+    }
     if (K > 0) {
       // -------------------------------------------- B': the short list
       // A threshold no higher than the k-th largest thread maximum leaves at
@@ -2280,38 +3247,7 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
             atomicAdd(&L.sh.tcnt[b], 1u);
           }
           __syncthreads();
-          if (tid < 64) {
-            constexpr int kPer = kTauBins / 64;
-            uint32_t cb[kPer];
-            uint32_t cs = 0u;
-#pragma unroll
-            for (int i = 0; i < kPer; ++i) {
-              cb[i] = L.sh.tcnt[kPer * tid + i];
-              cs += cb[i];
-            }
-            const uint32_t ic = wave_incl_scan(cs);
-            const uint64_t hit = __ballot(ic >= (uint32_t)K);
-            int bs = kTauBins;  // fewer than k threads hold a finite logit
-            if (hit) {
-              // first bin of each lane's run where the running count reaches
-              // k; lane f's is the answer
-              uint32_t acc = ic - cs;
-              int pos = kPer - 1;
-              bool found = false;
-#pragma unroll
-              for (int i = 0; i < kPer; ++i) {
-                acc += cb[i];
-                const bool h = !found && acc >= (uint32_t)K;
-                pos = h ? i : pos;
-                found = found || h;
-              }
-              const int f = __builtin_ctzll(hit);
-              bs = kPer * f + read_lane(pos, f);
-            }
-            if (tid == 0) L.misc[6] = bs;
-          }
-          __syncthreads();
-          const int bs = L.misc[6];
+          const int bs = find_count_bin(L, (uint32_t)K);
           // no bin reaches k: every finite token is a candidate
           tau = bs >= kTauBins ? kNegInf
                                : ((bs == kTauBins - 1 || sc == 0.0f) ? tlo
@@ -2472,7 +3408,7 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
           int w = 1;
           if (!last)
             w = started >= (uint32_t)G
-                    ? wait_exchange(ws, sync, (uint32_t)G, kClaimStats + (uint32_t)slice)
+                    ? wait_exchange(ws, sync, kArriveLists, (uint32_t)G, kClaimStats + (uint32_t)slice)
                     : 0;
           L.wait = w;
           L.last = last ? 1 : 0;
@@ -2582,13 +3518,11 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
       st_coherent_f64(&Ssum->z, zs);
     }
     if (MODE == kFused) {
-      // The exchange (a short-list row that fell back counts its second
-      // arrival).  The last arrival merges at once.  Another slice waits for
+      // The histograms' exchange.  The last arrival merges at once.  Another slice waits for
       // the rest only when every slice of the row has started, then claims
       // its own select; a slice that cannot wait, gives up, or finds its
       // select claimed leaves it to the last arriver.  Every slice that
       // merges computes the same cut (the merge is deterministic).
-      const uint32_t target = (uint32_t)(Krow > 0 ? 2 * G : G);
       drain_memory();
       __syncthreads();
       // Thread 0 arrives (the atomic returns the start count too); unless
@@ -2597,17 +3531,29 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
       // result is checked after the merge (the round trip overlaps the
       // merge's loads).  Same barriers as a plain wait.
       uint32_t claimed = 0u;
+      if (wide) {
+        // (a wide nucleus row: this slice's arrival at the first exchange
+        // was the last, or the last arriver has taken this histogram)
+        if (tid == 0) {
+          if ((n_word & kArriveMask) + 1u == (uint32_t)G) L.x1 = 1;
+          L.won = ((n_claim >> (kClaimStats + (uint32_t)slice)) & 1u) == 0u ? 1 : 0;
+        }
+        __syncthreads();
+        if (!L.won) return kJobLeave;
+      }
       if (tid == 0) {
         asm volatile("" ::"v"(tick));
         uint32_t* sync = row_sync(ws, row);
-        const uint32_t word = __hip_atomic_fetch_add(sync + kSyncArrive, 1u, __ATOMIC_RELAXED,
-                                                     __HIP_MEMORY_SCOPE_AGENT);
-        const uint32_t prev = word & kArriveMask, started = word >> 16;
-        const bool last = prev + 1u == target;
+        const uint32_t word = __hip_atomic_fetch_add(sync + kSyncArrive, 1u << kArriveHists,
+                                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint32_t prev = (word >> kArriveHists) & kArriveMask, started = word >> 16;
+        const bool last = prev + 1u == (uint32_t)G;
         if (last) L.xlast = 1;
         int w = 1;
         if (!last && !L.x1) {
-          w = started >= (uint32_t)G ? wait_exchange(ws, sync, target, (uint32_t)own) : 0;
+          w = started >= (uint32_t)G
+                  ? wait_exchange(ws, sync, kArriveHists, (uint32_t)G, (uint32_t)own)
+                  : 0;
           if (w == 1)
             claimed = __hip_atomic_fetch_or(sync + kSyncClaims, 1u << own, __ATOMIC_RELAXED,
                                             __HIP_MEMORY_SCOPE_AGENT);
@@ -2619,14 +3565,18 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
         // the first exchange's last arriver of a row that fell back builds
         // the histograms of the slices that left that exchange, then waits
         // (unless its arrival was the last) as any slice does
-        if (tid == 0) L.job = claim_next(row_sync(ws, row), G, own, kClaimStats, L.from_stats);
+        if (tid == 0) {
+          if (!L.stats_claimed) L.stats_left = claim_rest(row_sync(ws, row), G, own, kClaimStats);
+          L.stats_claimed = 1;
+          L.job = next_claimed(L.stats_left);
+        }
         __syncthreads();
         if (L.job >= 0) return next_job(kBehalfStats, L.job);
         if (tid == 0 && !L.xlast) {
           uint32_t* sync = row_sync(ws, row);
           // (claimed histograms took a while: the start count is read again)
           const int w = (ld_coherent(sync + kSyncArrive) >> 16) >= (uint32_t)G
-                            ? wait_exchange(ws, sync, target, (uint32_t)own)
+                            ? wait_exchange(ws, sync, kArriveHists, (uint32_t)G, (uint32_t)own)
                             : 0;
           if (w == 1)
             claimed = __hip_atomic_fetch_or(sync + kSyncClaims, 1u << own, __ATOMIC_RELAXED,
@@ -2637,7 +3587,7 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
       }
       if (!L.xlast && L.wait != 1) return kJobLeave;
       merge_stage(ws, P, row, c, L);
-      if (tid < 64) merge_wave<true>(ws, P, row, c, prm, L);
+      merge_bins<true>(ws, P, row, c, prm, L);
       if (tid == 0) L.won = (L.xlast || ((claimed >> own) & 1u) == 0u) ? 1 : 0;
       __syncthreads();
       if (!L.won) return kJobLeave;  // (the last arriver does this select)
@@ -2650,6 +3600,10 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
       if (!arrive_last(arrive, (uint32_t)G, &L.last)) return kJobLeave;
       if (K > 0 && short_gather<DT>(ws, P, row, c, prm, L)) {
         short_finish<DT>(ws, P, row, c, prm, L, rowp, mrow, K, lpp);
+        if (tid == 0) *arrive = 0u;
+        return kJobLeave;
+      }
+      if (nuc != 0 && nucleus_row<DT>(ws, P, row, c, prm, nuc, L, rowp, nullptr, lpp)) {
         if (tid == 0) *arrive = 0u;
         return kJobLeave;
       }
@@ -2883,7 +3837,11 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
   if (MODE != kFused) return kJobLeave;
   // the exchange's last arriver does the selects of the slices that left
   if (L.xlast) {
-    if (tid == 0) L.job = claim_next(row_sync(ws, row), G, own, 0u, L.from_select);
+    if (tid == 0) {
+      if (!L.select_claimed) L.select_left = claim_rest(row_sync(ws, row), G, own, 0u);
+      L.select_claimed = 1;
+      L.job = next_claimed(L.select_left);
+    }
     __syncthreads();
     if (L.job >= 0) return next_job(kSelectOnly, L.job);
   }
@@ -2894,22 +3852,22 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
 // work-group's own slice (with its start ticket), then whatever it claimed
 // for slices that left, and the departure; returns (thread 0) the row's
 // departure count before this one, for clear_if_last.
-template <int DT, int MODE, bool LP = false>
+template <int DT, int MODE, bool LP, bool NUC>
 __device__ __forceinline__ uint32_t run_task(const Workspace& ws, const SamplePlan& P, int row,
                                              int slice, TaskLds& L, const FusedLp& Lk) {
   if constexpr (MODE != kFused) {
-    (void)slice_job<DT, MODE, MODE, false>(ws, P, row, slice, L, slice, Lk);
+    (void)slice_job<DT, MODE, MODE, false, NUC>(ws, P, row, slice, L, slice, Lk);
     return 0u;
   } else {
     if (threadIdx.x == 0) {
       L.x1 = 0;
       L.xlast = 0;
-      L.from_stats = 0;
-      L.from_select = 0;
+      L.stats_claimed = 0;
+      L.select_claimed = 0;
     }
     // (no barrier: the job's first barriers come after its loads are issued,
     // before anything reads these)
-    int next = slice_job<DT, kFused, kFused, LP>(ws, P, row, slice, L, slice, Lk);
+    int next = slice_job<DT, kFused, kFused, LP, NUC>(ws, P, row, slice, L, slice, Lk);
     // (after the own pass: at most G - 1 claimed histograms and G claimed
     // selects; every thread returns the same job, read from LDS)
     for (int n = 0; n < 2 * kMaxSlices && next >= 0; ++n) {
@@ -2917,8 +3875,8 @@ __device__ __forceinline__ uint32_t run_task(const Workspace& ws, const SamplePl
       const int s = next & 0xff;
       __syncthreads();
       next = (next >> 8) == kBehalfStats
-                 ? slice_job<DT, kFused, kBehalfStats, LP>(ws, P, row, s, L, slice, Lk)
-                 : slice_job<DT, kFused, kSelectOnly, LP>(ws, P, row, s, L, slice, Lk);
+                 ? slice_job<DT, kFused, kBehalfStats, LP, NUC>(ws, P, row, s, L, slice, Lk)
+                 : slice_job<DT, kFused, kSelectOnly, LP, NUC>(ws, P, row, s, L, slice, Lk);
     }
     // (thread 0 has consumed its start ticket's result at the exchange)
     return threadIdx.x == 0 ? leave_row(ws, row) : 0u;
@@ -2944,7 +3902,7 @@ __global__ __launch_bounds__(kThreads) void k_fused(Workspace wsk, SamplePlan Pk
   const int slice = (int)blockIdx.x % G;
   if (ONE) {
     if (rowslot < P.rows) {
-      const uint32_t out = run_task<DT, kFused, LP>(ws, P, rowslot, slice, L, Lk);
+      const uint32_t out = run_task<DT, kFused, LP, true>(ws, P, rowslot, slice, L, Lk);
       if (threadIdx.x == 0) clear_if_last(ws, rowslot, G, out);
     }
     return;
@@ -3014,7 +3972,7 @@ __global__ __launch_bounds__(kThreads) void k_fused(Workspace wsk, SamplePlan Pk
     // the task holds a loop of its own)
     const int row = __builtin_amdgcn_readfirstlane(ordered ? (int)order[q] : q);
     const int slice_t = __builtin_amdgcn_readfirstlane((int)(t % (uint32_t)G));
-    pend_out = run_task<DT, kFused, LP>(wsr, Pr, row, slice_t, L, Lk);
+    pend_out = run_task<DT, kFused, LP, false>(wsr, Pr, row, slice_t, L, Lk);
     pend_row = row;
     __syncthreads();
   }
@@ -3028,14 +3986,14 @@ template <int DT>
 __global__ __launch_bounds__(kThreads) void k_stats(Workspace ws, SamplePlan P) {
   __shared__ TaskLds L;
   const FusedLp none{-1, nullptr, nullptr, nullptr, nullptr};
-  run_task<DT, kStatsOnly>(ws, P, (int)blockIdx.y, (int)blockIdx.x, L, none);
+  run_task<DT, kStatsOnly, false, true>(ws, P, (int)blockIdx.y, (int)blockIdx.x, L, none);
 }
 
 template <int DT>
 __global__ __launch_bounds__(kThreads) void k_select(Workspace ws, SamplePlan P) {
   __shared__ TaskLds L;
   const FusedLp none{-1, nullptr, nullptr, nullptr, nullptr};
-  run_task<DT, kSelectOnly>(ws, P, (int)blockIdx.y, (int)blockIdx.x, L, none);
+  run_task<DT, kSelectOnly, false, false>(ws, P, (int)blockIdx.y, (int)blockIdx.x, L, none);
 }
 
 template <int DT>
@@ -3045,7 +4003,7 @@ int launch_dt(const Workspace& ws, const SamplePlan& P, const FusedLp* lp, hipSt
     if (events) (void)hipEventRecord(reinterpret_cast<hipEvent_t>(events[i]), st);
   };
   mark(0);
-  if (P.fused) {
+  if (P.fused & kPlanFused) {
     const int rounds_rows = P.rows < P.rows_per_round ? P.rows : P.rows_per_round;
     const dim3 grid((unsigned)(rounds_rows * P.slices));
     const FusedLp none{-1, nullptr, nullptr, nullptr, nullptr};
@@ -3499,26 +4457,19 @@ int launch_verify_dt(const Workspace& ws, const VerifyPlan& Q, hipStream_t st) {
 
 }  // namespace
 
-int launch_verify_finish(const Workspace& ws, const VerifyPlan& Q, void* stream) {
-  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  switch (Q.dtype) {
-    case LSAMP_DTYPE_F32: return launch_verify_dt<LSAMP_DTYPE_F32>(ws, Q, st);
-    case LSAMP_DTYPE_BF16: return launch_verify_dt<LSAMP_DTYPE_BF16>(ws, Q, st);
-    default: return launch_verify_dt<LSAMP_DTYPE_F16>(ws, Q, st);
-  }
+template <int DT>
+int launch_verify_finish_dt(const Workspace& ws, const VerifyPlan& Q, void* stream) {
+  return launch_verify_dt<DT>(ws, Q, reinterpret_cast<hipStream_t>(stream));
 }
 
-int launch_sample(const Workspace& ws, const SamplePlan& P, const FusedLp* lp, void* stream,
-                  void* const* events) {
-  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  switch (P.dtype) {
-    case LSAMP_DTYPE_F32: return launch_dt<LSAMP_DTYPE_F32>(ws, P, lp, st, events);
-    case LSAMP_DTYPE_BF16: return launch_dt<LSAMP_DTYPE_BF16>(ws, P, lp, st, events);
-    default: return launch_dt<LSAMP_DTYPE_F16>(ws, P, lp, st, events);
-  }
+template <int DT>
+int launch_sample_dt(const Workspace& ws, const SamplePlan& P, const FusedLp* lp, void* stream,
+                     void* const* events) {
+  return launch_dt<DT>(ws, P, lp, reinterpret_cast<hipStream_t>(stream), events);
 }
 
-int set_spin_test(int32_t polls) {
+template <int DT>
+int set_spin_test_dt(int32_t polls) {
   return (int)hipMemcpyToSymbol(HIP_SYMBOL(g_spin_test), &polls, sizeof polls, 0,
                                 hipMemcpyHostToDevice);
 }
@@ -3541,12 +4492,11 @@ int fused_blocks_dt() {
   }
 }
 
-int fused_blocks_per_cu(int dtype) {
-  switch (dtype) {
-    case LSAMP_DTYPE_F32: return fused_blocks_dt<LSAMP_DTYPE_F32>();
-    case LSAMP_DTYPE_BF16: return fused_blocks_dt<LSAMP_DTYPE_BF16>();
-    default: return fused_blocks_dt<LSAMP_DTYPE_F16>();
-  }
-}
+// This file is compiled once per logits dtype (LSAMP_DT), side by side.
+template int launch_verify_finish_dt<LSAMP_DT>(const Workspace&, const VerifyPlan&, void*);
+template int launch_sample_dt<LSAMP_DT>(const Workspace&, const SamplePlan&, const FusedLp*, void*,
+                                        void* const*);
+template int set_spin_test_dt<LSAMP_DT>(int32_t);
+template int fused_blocks_dt<LSAMP_DT>();
 
 }  // namespace lsamp

@@ -1,0 +1,109 @@
+"""Rows of top-p / min-p alone in the one-round fused kernel: drawn from the
+slices' lists by the row's last arriver, or sent down the histogram path when
+the lists cannot decide them.  Every batch mixes rows of each outcome: nuclei
+of one token and of most of the row, one slice far above the others (its list
+ends above the row's cut), ties longer than a list, few or no tokens left by
+the mask, infinities and NaN.  Against the oracle, with the waits given up
+(every slice but a row's last arriver leaves) and without."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from common import compare, run_gpu, run_oracle
+from lsamp import _ffi
+from lsamp import workloads as W
+from lsamp.history import Cbv2RowState, TokenRing, csr, mlxlm_entries
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from lsamp.api import Context
+    c = Context(0, max_rows=256, max_vocab=262144)
+    yield c
+    c.close()
+
+
+def _bits(x, dtype):
+    if dtype == _ffi.DTYPE_F32:
+        return x.astype(np.float32)
+    if dtype == _ffi.DTYPE_F16:
+        return x.astype(np.float16).view(np.uint16)
+    return W.f32_to_bf16_bits(x.astype(np.float32))
+
+
+def _batch(rows, V, dtype, sem, seed, masked):
+    rng = np.random.default_rng(seed)
+    x = rng.normal(0, 3, (rows, V))
+    params, ents = [], []
+    for r in range(rows):
+        kind = r % 10
+        if kind == 1:  # a few tokens hold everything
+            x[r, rng.integers(0, V, 3)] += 25
+        elif kind == 2:  # close to flat: most of the row is kept
+            x[r] *= 0.25
+        elif kind == 3:  # one slice far above a broad rest
+            x[r, : V // 8] += 6
+            x[r, rng.integers(0, V // 8)] += 16
+        elif kind == 4:  # ties longer than any list
+            x[r] = np.round(2 * x[r]) / 2
+        elif kind == 5:
+            x[r, rng.integers(0, V, 5)] = -np.inf
+            x[r, rng.integers(0, V)] = np.nan
+        elif kind == 6:
+            x[r, [rng.integers(0, V), V - 1]] = np.inf
+        elif kind == 7:
+            x[r] = -np.inf
+            x[r, rng.integers(0, V, 2)] = 1.0
+        top_p = [0.9, 0.95, 0.5, 0.99, 1.0][r % 5]
+        min_p = [0.0, 0.0, 0.02, 0.3, 0.05][(r // 2) % 5]
+        T = [0.8, 1.0, 0.3, 1.7][(r // 3) % 4]
+        kw = dict(temperature=T, top_p=top_p, min_p=min_p if top_p < 1 else max(min_p, 0.1))
+        hist = rng.integers(0, V, 40).tolist() + np.argsort(-np.nan_to_num(x[r]))[:20].tolist()
+        if sem == _ffi.SEM_CBV2:
+            params.append(W.resolve_cbv2(presence_penalty=0.4, repetition_penalty=1.2, vocab=V, **kw))
+            ents.append(Cbv2RowState([], hist, 64, True, True, vocab=V).entries())
+        else:
+            params.append(W.resolve_mlxlm(repetition_penalty=1.2, repetition_context_size=64, **kw))
+            ring = TokenRing(64)
+            ring.load_prompt(hist)
+            ents.append(mlxlm_entries(repetition=ring))
+    row_ptr, entries = csr(ents)
+    cfg = dict(semantics=sem, dtype=dtype, rows=rows, vocab=V, logits=_bits(x, dtype),
+               params=W._params(params), row_ptr=row_ptr, entries=entries, bitmask=None,
+               mask_bits=0, uniforms=rng.random(rows, dtype=np.float32))
+    if masked:
+        allowed = rng.random((rows, (V + 31) // 32 * 32)) < \
+            np.array([1.1, 0.3, 0.001, 0.0])[np.arange(rows) % 4][:, None]
+        cfg["bitmask"] = np.packbits(allowed.reshape(rows, -1, 32)[:, :, ::-1], axis=2) \
+            .view(">u4").reshape(rows, -1).astype(np.uint32)
+        cfg["mask_bits"] = V
+    return cfg
+
+
+@pytest.mark.parametrize("rows,V,dtype,sem,masked", [
+    (200, 4099, _ffi.DTYPE_BF16, _ffi.SEM_CBV2, False),    # one slice a row
+    (120, 40003, _ffi.DTYPE_BF16, _ffi.SEM_MLXLM, False),  # two, unaligned rows
+    (80, 30720, _ffi.DTYPE_F16, _ffi.SEM_CBV2, True),      # three
+    (64, 65536, _ffi.DTYPE_F32, _ffi.SEM_CBV2, True),      # four
+    (60, 100000, _ffi.DTYPE_F32, _ffi.SEM_MLXLM, False),   # five: min-p alone
+    (20, 20480, _ffi.DTYPE_BF16, _ffi.SEM_CBV2, False),    # eight
+    (150, 70001, _ffi.DTYPE_F32, _ffi.SEM_CBV2, False),    # past one round
+])
+def test_rows_from_lists(ctx, rows, V, dtype, sem, masked):
+    cfg = _batch(rows, V, dtype, sem, rows + V, masked)
+    o = run_oracle(cfg, threads=16)
+    lib = _ffi.load_library()
+    compare(cfg, run_gpu(ctx, cfg), o, label="lists")
+    ctx.read_status()
+    _ffi.check(lib.lsamp_test_set_spin_limit(0, 16), "lsamp_test_set_spin_limit")
+    try:
+        g = run_gpu(ctx, cfg)
+    finally:
+        _ffi.check(lib.lsamp_test_set_spin_limit(0, 0), "lsamp_test_set_spin_limit")
+    ctx.read_status()
+    compare(cfg, g, o, label="lists, waits given up")
+    compare(cfg, run_gpu(ctx, cfg), o, label="lists again")
+    assert ctx.read_status() == 0
