@@ -9,8 +9,8 @@
 //
 // One 512-thread work-group owns one slice of one row and keeps the slice's
 // logits in registers (one pass over HBM):
-//   1. each thread takes its largest key (and, for log-probabilities, the
-//      sum of exp(x - m) over its logits, m its largest non-NaN logit);
+//   1. each thread takes its largest value, then that value's position in the
+//      one vector that holds it (and, for log-probabilities, the sum of exp(x - m) over its logits, m its largest non-NaN logit);
 //   2. tau = the k-th largest of the 512 thread maxima: a rank inside each
 //      wave (a count over the wave's 64 maxima in LDS), then a rank in the 8
 //      sorted wave lists (binary searches);
@@ -28,7 +28,10 @@
 // Work that only the few waves holding the candidates would run (unrolled
 // passes over their registers) is a long dependent chain with nothing to
 // overlap it, so the once-per-slice steps spread their work over all the
-// threads through LDS.
+// threads through LDS.  A CU is bound by its VALU work and by the slices'
+// latency chains, which the work-groups that share it overlap: 192 x 128,256
+// bf16, top 5: 32.4 us with 65,536-token slices and a packed (key, position)
+// a token, 21.4 us with three 32,768-token work-groups a CU (2.3 TB/s).
 #include <hip/hip_runtime.h>
 
 #include "lsamp_device.h"
@@ -133,17 +136,16 @@ __device__ __forceinline__ uint32_t negzero_bit(uint32_t b) {
   return b == RankBits<DT>::SIGN ? 1u : 0u;
 }
 
-constexpr int kRankCandCap = kRankMaxK * (rank_slice_len(kRankOptions - 1) / kThreads);
-
-// 16-byte vectors per thread of the largest slice
-constexpr int kRankMaxVecs = rank_slice_len(kRankOptions - 1) / kThreads / 4;
-
+// (sized by the slice, so that the small slices' work-groups share a CU)
+template <int OPT>
 struct alignas(16) RankLds {
+  static constexpr int kCandCap = kRankMaxK * (rank_slice_len(OPT) / kThreads);
+  static constexpr int kMaxVecs = rank_slice_len(OPT) / kThreads / 4;  // 16-byte vectors a thread
   union {
-    uint64_t cand[kRankCandCap];                // slice candidates (0-padded)
+    uint64_t cand[kCandCap];                    // slice candidates (0-padded)
     uint64_t lists[kRankMaxSlices][kRankMaxK];  // finalize: the slices' lists
   } u;
-  uint4 stage[kRankMaxK * kRankMaxVecs];  // logits of the threads at or above tau
+  uint4 stage[kRankMaxK * kMaxVecs];  // logits of the threads at or above tau
   int32_t stage_tid[kRankMaxK];
   uint64_t wt[kWaves][64];           // each wave's thread maxima
   uint64_t tops[kWaves][kRankMaxK];  // each wave's largest thread maxima (0-padded)
@@ -206,7 +208,8 @@ __global__ __launch_bounds__(kThreads) void k_rank(RankPlan P) {
   constexpr int SL = rank_slice_len(OPT);
   constexpr int Q = SL / (kThreads * N);  // 16-byte vectors per thread
   constexpr float kLog2e = 1.4426950408889634f;
-  __shared__ RankLds L;
+  __shared__ RankLds<OPT> L;
+  constexpr int kRankCandCap = RankLds<OPT>::kCandCap;
 
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int G = P.slices;
@@ -283,25 +286,69 @@ __global__ __launch_bounds__(kThreads) void k_rank(RankPlan P) {
     L.nstage = 0;
   }
 
-  // ---- 1. the thread's best key (and largest magnitude, for NaN / inf)
-  typename BT::T best = 0;
+  // ---- 1. the thread's best key (and largest magnitude, for NaN / inf).  The
+  // largest value is followed per vector with a copy of the first vector that
+  // holds it, so the position is looked for in one vector only: about 2.5
+  // operations a token, where a packed (key, position) per token took 10.
   uint32_t magmax = 0;
-  if (!tail) {
+  {
+    constexpr uint32_t M2 = B::W == 32 ? B::MAG : B::MAG * 0x10001u;
+    if constexpr (B::W == 32) {
 #pragma unroll
-    for (int q = 0; q < Q; ++q) {
+      for (int q = 0; q < Q; ++q)
+        magmax = max(max(max(magmax, r[q].x & M2), r[q].y & M2), max(r[q].z & M2, r[q].w & M2));
+    } else {
+      typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+      u16x2 m2 = {0, 0};
 #pragma unroll
-      for (int e = 0; e < N; ++e) {
-        const uint32_t b = elem_bits<DT>(r[q], e);
-        magmax = max(magmax, b & B::MAG);
-        const typename BT::T c = BT::pack(key_nn<DT>(b), q * N + e);
-        best = c > best ? c : best;
+      for (int q = 0; q < Q; ++q) {
+        m2 = __builtin_elementwise_max(m2, __builtin_bit_cast(u16x2, r[q].x & M2));
+        m2 = __builtin_elementwise_max(m2, __builtin_bit_cast(u16x2, r[q].y & M2));
+        m2 = __builtin_elementwise_max(m2, __builtin_bit_cast(u16x2, r[q].z & M2));
+        m2 = __builtin_elementwise_max(m2, __builtin_bit_cast(u16x2, r[q].w & M2));
       }
+      magmax = max((uint32_t)m2.x, (uint32_t)m2.y);
     }
   }
-  // a tail slice, or a thread that holds a NaN: again, NaN-aware and masked
-  const bool safe = tail || magmax > B::INF;
+  // places past the slice's tokens read -inf from here on (they come after
+  // the thread's own tokens, so the first maximum is a token's)
+  if (tail) {
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const int32_t rem = ns - (q * kThreads + tid) * N;
+      exclude_elems<DT>(r[q], ~0u << (uint32_t)(rem < 0 ? 0 : (rem > N ? N : rem)) &
+                                  ((1u << N) - 1u));
+    }
+  }
+  typename BT::T best = 0;
+  const bool safe = magmax > B::INF;  // a NaN: again, element by element
+  if (!safe && tid * N < ns) {
+    uint4 bv = r[0];
+    int bq = 0;
+    float bm = vec_max_nn<DT>(r[0]);
+#pragma unroll
+    for (int q = 1; q < Q; ++q) {
+      const float m = vec_max_nn<DT>(r[q]);
+      const bool up = m > bm;
+      bm = up ? m : bm;
+      bq = up ? q : bq;
+      bv.x = up ? r[q].x : bv.x;
+      bv.y = up ? r[q].y : bv.y;
+      bv.z = up ? r[q].z : bv.z;
+      bv.w = up ? r[q].w : bv.w;
+    }
+    int be = 0;
+    uint32_t bb = 0u;
+#pragma unroll
+    for (int e = N - 1; e >= 0; --e) {
+      const uint32_t b = elem_bits<DT>(bv, e);
+      const bool hit = bits_value<DT>(b) == bm;
+      be = hit ? e : be;
+      bb = hit ? b : bb;
+    }
+    best = BT::pack(key_nn<DT>(bb), bq * N + be);
+  }
   if (safe) {
-    best = 0;
     magmax = 0;
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
@@ -539,8 +586,7 @@ template <int DT>
 void launch_rank_dt(const RankPlan& P, hipStream_t st) {
   switch (P.option) {
     case 0: launch_rank_t<DT, 0>(P, st); break;
-    case 1: launch_rank_t<DT, 1>(P, st); break;
-    default: launch_rank_t<DT, 2>(P, st); break;
+    default: launch_rank_t<DT, 1>(P, st); break;
   }
 }
 
