@@ -161,6 +161,18 @@ void plan_slices(int32_t rows, int32_t vocab, int32_t slots, int32_t* slices, in
 int32_t nucleus_lists(int32_t dtype, int64_t tasks, int32_t slots) {
   return dtype == LSAMP_DTYPE_F32 || tasks <= slots ? kPlanLists : 0;
 }
+// Could a row go through lists?  (With no host copy of the parameters, yes;
+// a row that the copy misdescribes takes the histogram path.)
+bool any_nucleus(const lsamp_sample_args* a, int32_t slices) {
+  if (!a->params_host) return true;
+  for (int32_t r = 0; r < a->rows; ++r) {
+    const lsamp_row_params& p = a->params_host[r];
+    if (p.kind != LSAMP_KIND_FILTERED || (p.top_k > 0 && p.top_k < a->vocab)) continue;
+    const bool top_p = p.top_p < 1.0f && (a->semantics == LSAMP_SEM_CBV2 || p.top_p > 0.0f);
+    if (top_p ? slices <= kNucSlices : p.min_p > 0.0f) return true;
+  }
+  return false;
+}
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
@@ -296,7 +308,8 @@ lsamp_status lsamp::sample_step(const WorkspaceViews& v, const DeviceShape& d, i
   P.fused = !topk && mode != LSAMP_MODE_SPLIT && bpc > 0 && slots >= P.slices &&
             (!over || !(lp && lp->k >= 0));
   P.rows_per_round = P.fused && !over ? slots / P.slices : a->rows;
-  P.fused |= nucleus_lists(a->dtype, (int64_t)a->rows * P.slices, slots);
+  if (!topk && any_nucleus(a, P.slices))
+    P.fused |= nucleus_lists(a->dtype, (int64_t)a->rows * P.slices, slots);
   const size_t es = a->dtype == LSAMP_DTYPE_F32 ? 4 : 2;
   P.aligned = aligned16(a->logits) && ((size_t)a->row_stride * es) % 16 == 0;
   P.logits = a->logits;

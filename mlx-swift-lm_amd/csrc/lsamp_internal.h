@@ -309,8 +309,9 @@ int set_topk_spin_test(int32_t polls);  // the same hook for the top-k kernel's 
 constexpr uint32_t kStatusPenaltyCapacity = 2u;  // a verify position's entries did not fit
 
 // SamplePlan::fused: one kernel (else two), and rows of top-p / min-p alone go
-// through lists (nucleus rows).
+// through lists (nucleus rows; top-p rows of at most kNucSlices slices).
 constexpr int32_t kPlanFused = 1, kPlanLists = 2;
+constexpr int kNucSlices = 4;
 
 // Launch description resolved on the host.
 struct SamplePlan {

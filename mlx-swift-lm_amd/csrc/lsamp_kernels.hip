@@ -2217,7 +2217,6 @@ constexpr int kNucArea = kCandCap;             // keys of a row in each of two a
 static_assert(kMaxSlices * kKeptCap * sizeof(KeptItem) == kNucArea * sizeof(uint64_t),
               "cands and klist, both idle before the select phase");
 constexpr int kNucPer = 2 * kNucArea / kThreads;  // keys a thread of the last arriver holds
-constexpr int kNucSlices = 4;                  // top-p rows: at most this many slices
 constexpr int kNucFirst = 6;                   // of those, requested with the heads
 constexpr int kNucWaveQuads = (kQStage + 1) * kThreads / kWaves;  // quads a wave stages
 constexpr int kNucWaveKeys = kCandCap / kWaves;                   // keys a wave lists in LDS
@@ -3213,10 +3212,15 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
           if (L.last) {
             if (L.wait == 0 && nucleus_row<DT>(ws, P, row, c, prm, nuc, L, rowp, sync, lpp))
               return kJobLeave;
-            if (tid == 0) L.x1 = 1;
-          } else if (L.wait != (int)kVerdictHistogram) {
-            return kJobLeave;
+            // (its histogram from a re-read, as a claimed job: the registers
+            // need not hold the slice through the row's work above)
+            if (tid == 0) {
+              L.x1 = 1;
+              (void)claim_bit(sync, kClaimStats + (uint32_t)slice);
+            }
+            return next_job(kBehalfStats, slice);
           }
+          if (L.wait != (int)kVerdictHistogram) return kJobLeave;
           // (unless the last arriver has claimed this histogram)
           if (tid == 0) L.won = claim_bit(sync, kClaimStats + (uint32_t)slice) ? 1 : 0;
           __syncthreads();
@@ -3887,9 +3891,12 @@ __device__ __forceinline__ uint32_t run_task(const Workspace& ws, const SamplePl
 // ONE: a work-group per task (no loop over rounds, so nothing is hoisted out
 // of one and spilled before the first load): every row fits one round of the
 // grid, or (fp32) the grid is larger than the device.
+// NUC (with ONE): nucleus rows go through lists.  A batch whose host copy of the
+// parameters shows no such row runs the kernel without that code, which costs
+// the other rows 0.5 to 1.5 us by its registers and its size.
 // LP: raw log-probabilities in the same pass (lsamp_step); `Lk` is read
 // where it is used (the raw record and the finalize), not held throughout.
-template <int DT, bool ONE, bool LP>
+template <int DT, bool ONE, bool LP, bool NUC>
 __global__ __launch_bounds__(kThreads) void k_fused(Workspace wsk, SamplePlan Pk, FusedLp Lk) {
   __shared__ TaskLds L;
   // The kernel arguments are read in one round of scalar loads and held as
@@ -3902,7 +3909,7 @@ __global__ __launch_bounds__(kThreads) void k_fused(Workspace wsk, SamplePlan Pk
   const int slice = (int)blockIdx.x % G;
   if (ONE) {
     if (rowslot < P.rows) {
-      const uint32_t out = run_task<DT, kFused, LP, true>(ws, P, rowslot, slice, L, Lk);
+      const uint32_t out = run_task<DT, kFused, LP, NUC>(ws, P, rowslot, slice, L, Lk);
       if (threadIdx.x == 0) clear_if_last(ws, rowslot, G, out);
     }
     return;
@@ -4012,17 +4019,14 @@ int launch_dt(const Workspace& ws, const SamplePlan& P, const FusedLp* lp, hipSt
     // does not fit the registers.  The planner gives a batch past one round a
     // grid of one work-group per task, which the dispatcher starts in order as
     // work-groups end)
-    if constexpr (DT == LSAMP_DTYPE_F32) {
-      if (lp)
-        hipLaunchKernelGGL((k_fused<DT, true, true>), grid, dim3(kThreads), 0, st, ws, P, lk);
-      else
-        hipLaunchKernelGGL((k_fused<DT, true, false>), grid, dim3(kThreads), 0, st, ws, P, lk);
-    } else {
-      const bool one = P.rows <= P.rows_per_round;
-      auto kf = lp ? (one ? k_fused<DT, true, true> : k_fused<DT, false, true>)
-                   : (one ? k_fused<DT, true, false> : k_fused<DT, false, false>);
-      hipLaunchKernelGGL(kf, grid, dim3(kThreads), 0, st, ws, P, lk);
+    const bool nuc = (P.fused & kPlanLists) != 0;
+    auto kf = lp ? (nuc ? k_fused<DT, true, true, true> : k_fused<DT, true, true, false>)
+                 : (nuc ? k_fused<DT, true, false, true> : k_fused<DT, true, false, false>);
+    if constexpr (DT != LSAMP_DTYPE_F32) {
+      if (P.rows > P.rows_per_round)
+        kf = lp ? k_fused<DT, false, true, false> : k_fused<DT, false, false, false>;
     }
+    hipLaunchKernelGGL(kf, grid, dim3(kThreads), 0, st, ws, P, lk);
     mark(1);
   } else {
     const dim3 grid((unsigned)P.slices, (unsigned)P.rows);
@@ -4479,17 +4483,17 @@ int set_spin_test_dt(int32_t polls) {
 // and the grid is sized from this value.
 template <int DT>
 int fused_blocks_dt() {
-  int a = 0, b = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, k_fused<DT, true, false>, kThreads, 0) != hipSuccess)
-    return 0;
-  if constexpr (DT == LSAMP_DTYPE_F32) {
-    return a;  // (one round only)
-  } else {
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_fused<DT, false, false>, kThreads, 0) !=
-        hipSuccess)
-      return 0;
-    return a < b ? a : b;
-  }
+  int n = 0;
+  auto fits = [&n](auto kernel) {
+    int b = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, kernel, kThreads, 0) != hipSuccess) b = 0;
+    n = b < n ? b : n;
+  };
+  n = 1 << 20;
+  fits(k_fused<DT, true, false, true>);
+  fits(k_fused<DT, true, false, false>);
+  if constexpr (DT != LSAMP_DTYPE_F32) fits(k_fused<DT, false, false, false>);
+  return n;
 }
 
 // This file is compiled once per logits dtype (LSAMP_DT), side by side.
