@@ -2826,27 +2826,32 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
   if (mrow) load_mask_stage(mrow, P.mask_words, base32, end32, tid, ms);
   uint32_t* const mw = reinterpret_cast<uint32_t*>(L.sh.squad);
   static_assert(sizeof(L.sh.squad) >= kSliceWords * sizeof(uint32_t), "staged mask words fit");
-  // The slice's logits: 16-byte vectors all in flight at once, through one
-  // buffer descriptor over the slice (the lane's byte offset is fixed and
-  // the quad's is a scalar; lanes past the slice end read as zero, by the
-  // range check, until the exclusion pass).
+  // The slice's logits: 16-byte vectors through one buffer descriptor over the
+  // slice (the lane's byte offset is fixed and the quad's is a scalar; lanes
+  // past the slice end read as zero, by the range check, until the exclusion
+  // pass).  An unaligned row gets an empty range, so every load reads zero and
+  // the element-by-element path fills the slab in; the loads are issued
+  // either way, and every quad's without a branch, which keeps later waits
+  // exact.  Two banks go out here; the fp32 slab's other two each two banks
+  // ahead of the pass over them: with all of its 128 KB requested at once the
+  // waves sat in the issue of their loads until most of the slice had come,
+  // and only then began the pass (64 x 151,936: 6.7 us, then 5.3).
+  constexpr int NB = Slab<DT>::NB;
+  constexpr int kBanksAhead = 2;
   Slab<DT> S;
-  {
-    // (an unaligned row gets an empty range, so every load reads zero and
-    // the element-by-element path fills the slab in; the loads are issued
-    // either way, which keeps later waits exact)
-    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<char*>(rowp) + (size_t)base32 * ES, 0, aligned ? (end32 - base32) * ES : 0,
-        kBufferWord3);
-    const int lane_off = tid * 16;
-    // (every quad of the slab, without a branch: quads past the slice read
-    // zero, and straight-line loads let each later wait name its own quad)
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<char*>(rowp) + (size_t)base32 * ES, 0, aligned ? (end32 - base32) * ES : 0,
+      kBufferWord3);
+  auto load_bank = [&](int b) {
 #pragma unroll
-    for (int g = 0; g < Q; ++g) {
-      const auto w = __builtin_amdgcn_raw_buffer_load_b128(rs, lane_off, g * kThreads * 16, 0);
-      quad_set(S.bank[g / kQuadsPerBank], g % kQuadsPerBank, make_uint4(w[0], w[1], w[2], w[3]));
+    for (int s = 0; s < kQuadsPerBank; ++s) {
+      const auto w = __builtin_amdgcn_raw_buffer_load_b128(
+          rs, tid * 16, (b * kQuadsPerBank + s) * kThreads * 16, 0);
+      quad_set(S.bank[b], s, make_uint4(w[0], w[1], w[2], w[3]));
     }
-  }
+  };
+#pragma unroll
+  for (int b = 0; b < kBanksAhead && b < NB; ++b) load_bank(b);
   // (fused, own slice) the row's start ticket, issued after the slice's
   // loads so that their waits do not include it; its result is consumed at
   // the first exchange, before the arrival
@@ -2867,24 +2872,25 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
   float emax = kNegInf;  // this thread's patched entry values
   if (mrow) store_mask_stage(ms, P.mask_words, P.mask_bits, P.mask_tail, base32, end32, tid, mw);
   mark_slice_entries<DT>(P, c, prm, mrow, rowp, base, end, se, ep, tid, em, emax);
-  if (!aligned || (end32 & (N - 1)) != 0) {
-    // unaligned rows, or the row's last partial quad: element by element
-    // (after the entry bitmap, whose wait these loads would otherwise delay)
-    for_quads(S, nq, [&](int g, uint4& v) -> bool {
-      const int32_t i0 = base32 + (tid + g * kThreads) * N;
-      if (i0 >= end32 || (aligned && i0 + N <= end32)) return false;
-      uint32_t b[N];
+  // unaligned rows, or the row's last partial quad: element by element (after
+  // the entry bitmap, whose wait these loads would otherwise delay)
+  const bool fill = !aligned || (end32 & (N - 1)) != 0;
+  auto fill_bank = [&](int b) {
+    const int n = nq - b * kQuadsPerBank;
+#pragma unroll 1
+    for (int s = 0; s < (n < kQuadsPerBank ? n : kQuadsPerBank); ++s) {
+      const int32_t i0 = base32 + (tid + (b * kQuadsPerBank + s) * kThreads) * N;
+      if (i0 >= end32 || (aligned && i0 + N <= end32)) continue;
+      uint32_t x[N];
 #pragma unroll
-      for (int e = 0; e < N; ++e) b[e] = i0 + e < end32 ? load_raw_bits<DT>(rowp, i0 + e) : 0u;
-      if constexpr (N == 4) {
-        v = make_uint4(b[0], b[1], b[2], b[3]);
-      } else {
-        v = make_uint4(b[0] | (b[1] << 16), b[2] | (b[3] << 16), b[4] | (b[5] << 16),
-                       b[6] | (b[7] << 16));
-      }
-      return true;
-    });
-  }
+      for (int e = 0; e < N; ++e) x[e] = i0 + e < end32 ? load_raw_bits<DT>(rowp, i0 + e) : 0u;
+      if constexpr (N == 4)
+        quad_set(S.bank[b], s, make_uint4(x[0], x[1], x[2], x[3]));
+      else
+        quad_set(S.bank[b], s, make_uint4(x[0] | (x[1] << 16), x[2] | (x[3] << 16),
+                                          x[4] | (x[5] << 16), x[6] | (x[7] << 16)));
+    }
+  };
 
   // Masked tokens, tokens of the entry table (their patched values live in
   // L.ex) and lanes past the slice end become -inf in the register copy, and
@@ -2926,7 +2932,7 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
   float zt = 0.0f, nbz = __FLT_MAX__;
   // (LP, own pass) the raw logits' statistics, before any exclusion
   RawAcc ra{kNegInf, 0.0f, __FLT_MAX__, 0u};
-  for_quads_static(S, nq, [&](int g, uint4& v) -> bool {
+  auto first_pass = [&](int g, uint4& v) {
     const int32_t i0 = base32 + (tid + g * kThreads) * N;
     const uint32_t pcur = pw;
     if (g + 1 < Q) pw = penw[(g + 1) * kQuadWords];
@@ -2937,8 +2943,7 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
     if constexpr (LP && JM == kFused) raw_add<DT>(ra, v, tail & FULL, probe);
     uint32_t ex = ((pcur >> pen_shift) | tail) & FULL;
     if (mrow) ex |= ~staged_allow_bits(mw, i0 - base32, N) & FULL;
-    // (NaNs are rare, behind a branch; entry tokens are in most quads of a
-    // wave, so the exclusion runs unconditionally, a no-op without bits)
+    // (NaNs are rare, behind a branch)
     if (nonfinite_seen<DT>(probe)) {
 #pragma unroll
       for (int e = 0; e < N; ++e) {
@@ -2946,7 +2951,7 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
         if (x != x) ex |= 1u << e;
       }
     }
-    exclude_elems<DT>(v, ex);
+    if (__ballot(ex != 0u) != 0ull) exclude_elems<DT>(v, ex);
     if (jm != kSelectOnly) {
       const float qm = vec_max_nn<DT>(v);  // NaNs are excluded by now
       if constexpr (kKeepQm) qmc[g * kThreads + tid] = qm;
@@ -2964,8 +2969,20 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
           zt += __builtin_amdgcn_exp2f(__builtin_fmaf(vec_elem<DT>(v, e), lgz, nbz));
       }
     }
-    return true;
-  });
+  };
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    if (b + kBanksAhead < NB) load_bank(b + kBanksAhead);
+    if (fill) fill_bank(b);
+#pragma unroll
+    for (int s = 0; s < kQuadsPerBank; ++s) {
+      if (b * kQuadsPerBank + s < nq) {
+        uint4 v = quad_get(S.bank[b], s);
+        first_pass(b * kQuadsPerBank + s, v);
+        quad_set(S.bank[b], s, v);
+      }
+    }
+  }
   const bool zref = nbz < __FLT_MAX__;
   finish_slice_entries<DT>(P, c, prm, mrow, se, ep, em, emax);
   xmax = __builtin_fmaxf(xmax, emax);
