@@ -161,31 +161,41 @@ void plan_slices(int32_t rows, int32_t vocab, int32_t slots, int32_t* slices, in
 int32_t nucleus_lists(int32_t dtype, int64_t tasks, int32_t slots) {
   return dtype == LSAMP_DTYPE_F32 || tasks <= slots ? kPlanLists : 0;
 }
-// Could a row go through lists?  (With no host copy of the parameters, yes;
-// a row that the copy misdescribes takes the histogram path.)
-bool any_nucleus(const lsamp_sample_args* a, int32_t slices) {
-  if (!a->params_host) return true;
+// What the host copy of the parameters shows of a batch's rows (without one:
+// that every row may be anything).
+struct RowMix {
+  bool nucleus;  // some row could go through a nucleus list
+  bool lists;    // at least half of the rows are drawn from lists of some kind
+};
+RowMix row_mix(const lsamp_sample_args* a, int32_t slices) {
+  if (!a->params_host) return RowMix{true, true};
+  int32_t nucleus = 0, brief = 0;
   for (int32_t r = 0; r < a->rows; ++r) {
     const lsamp_row_params& p = a->params_host[r];
-    if (p.kind != LSAMP_KIND_FILTERED || (p.top_k > 0 && p.top_k < a->vocab)) continue;
+    const bool top_k = p.top_k > 0 && p.top_k < a->vocab;
     const bool top_p = p.top_p < 1.0f && (a->semantics == LSAMP_SEM_CBV2 || p.top_p > 0.0f);
-    if (top_p ? slices <= kNucSlices : p.min_p > 0.0f) return true;
+    if (p.kind == LSAMP_KIND_ARGMAX || !(p.temperature > 0.0f && p.temperature < INFINITY) ||
+        (p.kind == LSAMP_KIND_FILTERED && top_k && p.top_k <= kShortMaxK))
+      ++brief;
+    else if (p.kind == LSAMP_KIND_FILTERED && !top_k &&
+             (top_p ? slices <= kNucSlices : p.min_p > 0.0f))
+      ++nucleus;
   }
-  return false;
+  return RowMix{nucleus > 0, 2 * (nucleus + brief) >= a->rows};
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // Slice option of a ranking launch: 16,384-token slices, or 32,768 where a row
-// would have more than 8 (the merge of its lists is then twice as wide: 32 x
-// 151,936 bf16 top-2 11.0 us against 9.9), or where 16-bit rows make at least
+// would have more than 8 (fp32: 12; the merge of its lists is then twice as
+// wide: 32 x 151,936 bf16 top-2 11.0 us against 9.9), or where 16-bit rows make at least
 // three quarters of a work-group per CU of them anyway, most of a slice full
 // (192 x 128,256 log-probabilities 28.5 us against 21.4; fp32 rows, twice the
 // registers, gain nothing: 128 x 128,256 23.2 against 27.5).
 void plan_rank(int32_t rows, int32_t vocab, int32_t dtype, int32_t cus, int32_t* option,
                int32_t* slices) {
   const auto count = [vocab](int o) { return (vocab + rank_slice_len(o) - 1) / rank_slice_len(o); };
-  const bool wide = count(0) > 8 ||
+  const bool wide = count(0) > (dtype == LSAMP_DTYPE_F32 ? 12 : 8) ||
                     (dtype != LSAMP_DTYPE_F32 && vocab > rank_slice_len(1) * 3 / 4 &&
                      (int64_t)rows * count(1) >= (int64_t)cus * 3 / 4);
   *option = wide ? 1 : 0;
@@ -302,13 +312,17 @@ lsamp_status lsamp::sample_step(const WorkspaceViews& v, const DeviceShape& d, i
   // built for the fp32 slab: it would not fit the registers) runs the one-round
   // kernel over a grid larger than the device: its hand-off assumes no
   // co-residency, so the dispatcher's own order serves.  128 rows x 151,936
-  // with top-p: 94 us, the split kernels (which read every slice twice) 102.
-  // With raw log-probabilities asked for, such a batch keeps the split kernels.
+  // with top-p: 71 us, the split kernels (which read every slice twice) 101.
+  // A batch most of whose rows exchange histograms keeps the split kernels
+  // (193 rows x 32,000 without filters: 131 us, 161 in one kernel, whose
+  // slices wait for each other), and so does one that asks for raw
+  // log-probabilities.
   const bool over = a->dtype == LSAMP_DTYPE_F32 && (int64_t)a->rows * P.slices > slots;
+  const RowMix mix = row_mix(a, P.slices);
   P.fused = !topk && mode != LSAMP_MODE_SPLIT && bpc > 0 && slots >= P.slices &&
-            (!over || !(lp && lp->k >= 0));
+            (!over || (mix.lists && !(lp && lp->k >= 0)));
   P.rows_per_round = P.fused && !over ? slots / P.slices : a->rows;
-  if (!topk && any_nucleus(a, P.slices))
+  if (!topk && mix.nucleus)
     P.fused |= nucleus_lists(a->dtype, (int64_t)a->rows * P.slices, slots);
   const size_t es = a->dtype == LSAMP_DTYPE_F32 ? 4 : 2;
   P.aligned = aligned16(a->logits) && ((size_t)a->row_stride * es) % 16 == 0;

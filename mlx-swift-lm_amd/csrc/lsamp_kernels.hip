@@ -342,16 +342,26 @@ static_assert(kSelQueue >= kThreads / kWaves * 8, "a quad step of a wave fits th
 // trips), else 256 (one).  A cut in those bins needs no further round trip.
 // Whole work-group.
 constexpr int kMergeStageBins = 512;
+// A row without filters keeps every token: unless its statistics are wanted,
+// only its maximum is needed ahead of the select, no histogram.
+__device__ __forceinline__ bool open_row(const SamplePlan& P, const RowCtx& c,
+                                         const lsamp_row_params& prm) {
+  if (c.kind == LSAMP_KIND_ARGMAX || P.stats) return false;
+  return c.kind == LSAMP_KIND_CATEGORICAL ||
+         (!(prm.top_k > 0 && prm.top_k < P.vocab) && !(prm.min_p > 0.0f) &&
+          top_p_limit(P, c, prm, 1.0) < 0.0);
+}
 __device__ __forceinline__ int merge_stage_batches(int slices) { return slices > 4 ? 2 : 1; }
 __device__ __forceinline__ void merge_stage(const Workspace& ws, const SamplePlan& P, int row,
-                                            const RowCtx& c, TaskLds& L) {
+                                            const RowCtx& c, const lsamp_row_params& prm,
+                                            TaskLds& L) {
   constexpr int kPer = kMergeStageBins / 64;
   static_assert(kMergeStageBins <= kBins, "the staged bins fit the merge arrays");
   static_assert(kWaves >= kMaxSlices, "a wave per slice");
   const int tid = fresh_tid(), l = tid & 63, wv = tid >> 6;
   const int G = P.slices;
   const SliceSummary* summ = ws.summaries + (size_t)row * kMaxSlices;
-  const bool hist_row = c.kind != LSAMP_KIND_ARGMAX;
+  const bool hist_row = c.kind != LSAMP_KIND_ARGMAX && !open_row(P, c, prm);
   int32_t ht = 0, hn = 0;
   if (l < G) {
     ht = ld_coherent(&summ[l].top_bin);
@@ -408,7 +418,7 @@ __device__ __forceinline__ void merge_bins(const Workspace& ws, const SamplePlan
   const int G = P.slices;
   const int64_t V = P.vocab;
   const SliceSummary* summ = ws.summaries + (size_t)row * kMaxSlices;
-  const bool hist_row = c.kind != LSAMP_KIND_ARGMAX;
+  const bool hist_row = c.kind != LSAMP_KIND_ARGMAX && !open_row(P, c, prm);
   constexpr int kBlk = 4;  // blocks of 64 bins per batch
   // (STAGED: merge_stage has the heads in LDS and the top staged_batches
   // batches of bins aligned there)
@@ -475,6 +485,8 @@ __device__ __forceinline__ void merge_bins(const Workspace& ws, const SamplePlan
     // token) is a candidate and the finalize keeps the first in id order
     info.cut = 0;
     info.count_above = 0;
+  } else if (info.mode == kModeNormal && !hist_row) {
+    info.count_above = 0x7fffffff;  // (the slices did not count)
   } else if (info.mode == kModeNormal) {
     const double inv_frac = 1.0 / (double)(1ull << kMassFracBits);
     // total mass relative to the row top: each slice's total is relative to
@@ -3456,7 +3468,7 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
     }
 
     // ------------------------------------------------ B: histogram
-    const bool want_hist = has_finite && c.kind != LSAMP_KIND_ARGMAX;
+    const bool want_hist = has_finite && c.kind != LSAMP_KIND_ARGMAX && !open_row(P, c, prm);
     if (want_hist) {
       const float tail_edge = (float)(top - kBins + 1);
       // Branch-free per token (excluded tokens add zero to a discard word of
@@ -3607,7 +3619,7 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
         __syncthreads();
       }
       if (!L.xlast && L.wait != 1) return kJobLeave;
-      merge_stage(ws, P, row, c, L);
+      merge_stage(ws, P, row, c, prm, L);
       merge_bins<true>(ws, P, row, c, prm, L);
       if (tid == 0) L.won = (L.xlast || ((claimed >> own) & 1u) == 0u) ? 1 : 0;
       __syncthreads();

@@ -10,7 +10,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from common import compare, run_gpu, run_oracle
+from common import compare, run_gpu, run_oracle, to_torch_logits
 from lsamp import _ffi
 from lsamp import workloads as W
 from lsamp.history import Cbv2RowState, TokenRing, csr, mlxlm_entries
@@ -106,4 +106,34 @@ def test_rows_from_lists(ctx, rows, V, dtype, sem, masked):
     ctx.read_status()
     compare(cfg, g, o, label="lists, waits given up")
     compare(cfg, run_gpu(ctx, cfg), o, label="lists again")
+    assert ctx.read_status() == 0
+
+
+@pytest.mark.parametrize("rows,V,dtype", [
+    (7, 4099, _ffi.DTYPE_BF16),    # unaligned rows
+    (64, 65536, _ffi.DTYPE_F32),   # one round
+    (150, 40003, _ffi.DTYPE_F16),  # several rounds
+    (150, 70001, _ffi.DTYPE_F32),  # past one round: split
+])
+def test_rows_without_filters(ctx, rows, V, dtype):
+    """Every token is kept, so without statistics no histogram is built: the
+    tokens are those of the call with statistics, which the oracle checks."""
+    cfg = _batch(rows, V, dtype, _ffi.SEM_CBV2, rows + V, False)
+    for r in range(rows):
+        if r % 3:
+            cfg["params"][r] = W._params([W.resolve_cbv2(
+                temperature=[0.8, 1.0, 0.3, 1.7][r % 4], presence_penalty=0.4,
+                repetition_penalty=1.2, vocab=V)])[0]
+    full = run_gpu(ctx, cfg)
+    compare(cfg, full, run_oracle(cfg, threads=16), label="no filters")
+    for mode in (_ffi.MODE_AUTO, _ffi.MODE_SPLIT):
+        ctx.set_mode(mode)
+        try:
+            out = ctx.sample(to_torch_logits(cfg), cfg["params"], semantics=cfg["semantics"],
+                             vocab=V, row_ptr=cfg["row_ptr"], entries=cfg["entries"],
+                             uniforms=cfg["uniforms"])
+        finally:
+            ctx.set_mode(_ffi.MODE_AUTO)
+        assert np.array_equal(out["tokens"].cpu().numpy(), full["tokens"])
+        assert np.array_equal(out["row_flags"].cpu().numpy().astype(np.uint32), full["row_flags"])
     assert ctx.read_status() == 0
