@@ -191,11 +191,14 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 // wide: 32 x 151,936 bf16 top-2 11.0 us against 9.9), or where 16-bit rows make at least
 // three quarters of a work-group per CU of them anyway, most of a slice full
 // (192 x 128,256 log-probabilities 28.5 us against 21.4; fp32 rows, twice the
-// registers, gain nothing: 128 x 128,256 23.2 against 27.5).
-void plan_rank(int32_t rows, int32_t vocab, int32_t dtype, int32_t cus, int32_t* option,
-               int32_t* slices) {
+// registers, gain nothing: 128 x 128,256 23.2 against 27.5).  Without a top k
+// there are no lists to merge: small slices while two work-groups a CU hold the
+// grid (6 x 151,936 chosen log-probability 6.2 us against 7.5).
+void plan_rank(int32_t rows, int32_t vocab, int32_t dtype, int32_t k, int32_t cus,
+               int32_t* option, int32_t* slices) {
   const auto count = [vocab](int o) { return (vocab + rank_slice_len(o) - 1) / rank_slice_len(o); };
-  const bool wide = count(0) > (dtype == LSAMP_DTYPE_F32 ? 12 : 8) ||
+  const bool lists = k > 0 || (int64_t)rows * count(0) > 2 * (int64_t)cus;
+  const bool wide = (lists && count(0) > (dtype == LSAMP_DTYPE_F32 ? 12 : 8)) ||
                     (dtype != LSAMP_DTYPE_F32 && vocab > rank_slice_len(1) * 3 / 4 &&
                      (int64_t)rows * count(1) >= (int64_t)cus * 3 / 4);
   *option = wide ? 1 : 0;
@@ -218,7 +221,7 @@ lsamp_status rank_common(lsamp_context* ctx, RankPlan& P, int32_t min_vocab, voi
   if (!P.logits) return fail(LSAMP_ERR_INVALID_ARGUMENT, "logits is NULL");
   const size_t es = P.dtype == LSAMP_DTYPE_F32 ? 4 : 2;
   P.vec = P.col_stride == 1 && aligned16(P.logits) && ((size_t)P.row_stride * es) % 16 == 0;
-  plan_rank(P.rows, P.vocab, P.dtype, ctx->cus, &P.option, &P.slices);
+  plan_rank(P.rows, P.vocab, P.dtype, P.k, ctx->cus, &P.option, &P.slices);
   P.part = ctx->rank_part;
   P.arrive = ctx->arrive_rank;
   DeviceGuard guard(ctx->device);
