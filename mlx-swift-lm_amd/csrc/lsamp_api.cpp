@@ -193,12 +193,14 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 // (192 x 128,256 log-probabilities 28.5 us against 21.4; fp32 rows, twice the
 // registers, gain nothing: 128 x 128,256 23.2 against 27.5).  Without a top k
 // there are no lists to merge: small slices while two work-groups a CU hold the
-// grid (6 x 151,936 chosen log-probability 6.2 us against 7.5).
+// grid (6 x 151,936 chosen log-probability 6.2 us against 7.5).  A row never has
+// more than kRankMaxSlices of them: its records and arrivals are sized for that.
 void plan_rank(int32_t rows, int32_t vocab, int32_t dtype, int32_t k, int32_t cus,
                int32_t* option, int32_t* slices) {
   const auto count = [vocab](int o) { return (vocab + rank_slice_len(o) - 1) / rank_slice_len(o); };
   const bool lists = k > 0 || (int64_t)rows * count(0) > 2 * (int64_t)cus;
-  const bool wide = (lists && count(0) > (dtype == LSAMP_DTYPE_F32 ? 12 : 8)) ||
+  const bool wide = count(0) > kRankMaxSlices ||
+                    (lists && count(0) > (dtype == LSAMP_DTYPE_F32 ? 12 : 8)) ||
                     (dtype != LSAMP_DTYPE_F32 && vocab > rank_slice_len(1) * 3 / 4 &&
                      (int64_t)rows * count(1) >= (int64_t)cus * 3 / 4);
   *option = wide ? 1 : 0;
@@ -521,6 +523,17 @@ lsamp_status lsamp_test_set_spin_limit(int32_t device, int32_t polls) {
   if (set_spin_test(polls) != 0 || set_topk_spin_test(polls) != 0 ||
       hipDeviceSynchronize() != hipSuccess)
     return fail(LSAMP_ERR_DEVICE, "setting the wait test hook failed");
+  return ok();
+}
+
+lsamp_status lsamp_test_plan_rank(int32_t rows, int32_t vocab, int32_t dtype, int32_t k,
+                                  int32_t cus, int32_t* slices, int32_t* slice_len) {
+  if (!slices || !slice_len) return fail(LSAMP_ERR_INVALID_ARGUMENT, "NULL argument");
+  if (rows <= 0 || vocab <= 0 || vocab > kMaxVocab || cus <= 0)
+    return fail(LSAMP_ERR_SHAPE, "rows %d / vocab %d / cus %d invalid", rows, vocab, cus);
+  int32_t option = 0;
+  plan_rank(rows, vocab, dtype, k, cus, &option, slices);
+  *slice_len = rank_slice_len(option);
   return ok();
 }
 

@@ -213,3 +213,19 @@ def test_rng_uniform_matches_the_oracle(lib):
         k = int(rng.integers(0, 2**63, dtype=np.uint64))
         for purpose in (0, 1, 7):
             assert lib.lsamp_rng_uniform(k, purpose) == O.rng_uniform(k, purpose)
+
+
+@pytest.mark.parametrize("dtype", [_ffi.DTYPE_F32, _ffi.DTYPE_BF16, _ffi.DTYPE_F16])
+def test_ranking_slices_fit_their_records(lib, dtype):
+    """The ranking keeps 16 slice records a row: no plan makes more slices, and
+    the slices cover the row, from one token to the largest vocabulary."""
+    g, n = ctypes.c_int32(), ctypes.c_int32()
+    vocabs = sorted({1, 2, 4099, 248320, 524288} |
+                    {16384 * i + d for i in range(1, 32) for d in (-1, 0, 1)})
+    for vocab in vocabs:
+        for rows in (1, 2, 6, 13, 16, 64, 114, 192, 256, 1024):
+            for k in (0, 1, 2, 5, 32):
+                _ffi.check(lib.lsamp_test_plan_rank(rows, vocab, dtype, k, 256, ctypes.byref(g),
+                                                    ctypes.byref(n)), "lsamp_test_plan_rank")
+                assert 1 <= g.value <= 16, (rows, vocab, k, g.value)
+                assert (g.value - 1) * n.value < vocab <= g.value * n.value, (rows, vocab, k)

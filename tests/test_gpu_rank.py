@@ -157,3 +157,24 @@ def test_argument_errors(ctx):
         ctx.top2(x[:, :1])
     with pytest.raises(_ffi.LsampError):
         ctx.top2(torch.zeros((65, 100), dtype=torch.bfloat16, device="cuda"))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("vocab", [262145, 300001, 524288])
+def test_chosen_log_probability_of_the_largest_vocabularies(vocab, dtype):
+    """Without a top k the ranking keeps its small slices on small grids, but
+    never more of them than a row has records for (16)."""
+    import torch
+    from lsamp.api import Context
+    rng = np.random.default_rng(vocab + dtype)
+    rows = 3
+    c = Context(0, max_rows=rows, max_vocab=vocab)
+    try:
+        b = batch(rng, rows, vocab, dtype, specials=False)
+        tok = np.array([0, vocab // 2, vocab - 1], np.int32)
+        for _ in range(2):  # (the arrival counters return to zero)
+            check_logprobs(c, b, dtype, rows, vocab, vocab, 1, 0, tokens=tok, label="no top k")
+        check_logprobs(c, b, dtype, rows, vocab, vocab, 1, 5, tokens=tok, label="top 5")
+    finally:
+        torch.cuda.synchronize()
+        c.close()
