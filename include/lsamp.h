@@ -357,9 +357,9 @@ lsamp_status lsamp_context_read_status(lsamp_context* ctx, uint32_t* bits);
 /* Launch shape of the context's last lsamp_sample call (diagnostics; no
  * device work): fused with raw log-probabilities (4, lsamp_step), top-k with
  * raw log-probabilities (3, lsamp_step), top-k (2), fused on a grid that fits
- * the device at once (1), or more work-groups than that (0: the split kernels,
- * or the fused kernel's fp32 batches past one round), slices per row, tokens per slice, rows per round of the fused grid,
- * work-groups per kernel launch. */
+ * the device at once (1), fused on a larger grid (5: fp32 batches), split
+ * kernels (0); slices per row, tokens per slice, rows per round of the fused
+ * grid, work-groups per kernel launch. */
 typedef struct lsamp_launch_info {
   int32_t fused;
   int32_t slices;

@@ -27,6 +27,11 @@ lsamp_status lsamp_test_set_spin_limit(int32_t device, int32_t polls);
 lsamp_status lsamp_test_plan_rank(int32_t rows, int32_t vocab, int32_t dtype, int32_t k,
                                   int32_t cus, int32_t* slices, int32_t* slice_len);
 
+/* For each of the first `rows` rows of the context's last sampling or
+ * verification launch (not the top-k kernel's): 1 when the row was drawn from
+ * its slices' lists, 0 when it took the histogram path.  Synchronous. */
+lsamp_status lsamp_test_rows_from_lists(lsamp_context* ctx, int32_t rows, int32_t* out);
+
 #ifdef __cplusplus
 }
 #endif

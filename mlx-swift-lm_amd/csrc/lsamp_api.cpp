@@ -11,6 +11,7 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <vector>
 
 #include "lsamp_internal.h"
 #include "../../include/lsamp_testing.h"
@@ -389,7 +390,11 @@ lsamp_status lsamp::sample_step(const WorkspaceViews& v, const DeviceShape& d, i
     flp.ids = lp->ids;
     flp.rec = v.rawrec;
   }
-  last->fused = topk ? (lp_fused ? 3 : 2) : (lp_sample ? 4 : (over ? 0 : P.fused & kPlanFused));
+  last->fused = topk                          ? (lp_fused ? 3 : 2)
+                : lp_sample                   ? 4
+                : !(P.fused & kPlanFused)     ? 0
+                : over                        ? 5
+                                              : 1;
   last->slices = P.slices;
   last->slice_len = P.slice_len;
   last->rows_per_round = P.rows_per_round;
@@ -534,6 +539,20 @@ lsamp_status lsamp_test_plan_rank(int32_t rows, int32_t vocab, int32_t dtype, in
   int32_t option = 0;
   plan_rank(rows, vocab, dtype, k, cus, &option, slices);
   *slice_len = rank_slice_len(option);
+  return ok();
+}
+
+lsamp_status lsamp_test_rows_from_lists(lsamp_context* ctx, int32_t rows, int32_t* out) {
+  if (!ctx || !out) return fail(LSAMP_ERR_INVALID_ARGUMENT, "NULL argument");
+  if (rows <= 0 || rows > ctx->ws.max_rows)
+    return fail(LSAMP_ERR_SHAPE, "rows %d outside [1, %d]", rows, ctx->ws.max_rows);
+  DeviceGuard guard(ctx->device);
+  std::vector<RowInfo> info((size_t)rows);
+  if (hipDeviceSynchronize() != hipSuccess ||
+      hipMemcpy(info.data(), ctx->ws.rows, info.size() * sizeof(RowInfo),
+                hipMemcpyDeviceToHost) != hipSuccess)
+    return fail(LSAMP_ERR_DEVICE, "reading the row decisions failed");
+  for (int32_t r = 0; r < rows; ++r) out[r] = info[(size_t)r].done;
   return ok();
 }
 

@@ -104,7 +104,7 @@ struct RowInfo {
   double z;             // sum exp(q - q_top) over every finite token
   double p_limit;       // top-p comparison bound (top_p * z), < 0 if off
   int32_t kept_cands;   // select finalize: kept candidates, listed first in cands[row]
-  int32_t done;         // split mode: the stats kernel already drew this row's token
+  int32_t done;         // 1: drawn from lists (split mode: by the stats kernel already)
 };
 
 // Per-slice partial results of the select phase.

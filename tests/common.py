@@ -116,6 +116,15 @@ def compare(cfg, gpu, ora, *, label="", uniforms=None):
     return boundary_rows
 
 
+def rows_from_lists(ctx, rows):
+    """Which of the last launch's rows were drawn from their slices' lists."""
+    import ctypes
+    out = (ctypes.c_int32 * rows)()
+    _ffi.check(ctx.lib.lsamp_test_rows_from_lists(ctx.handle, rows, out),
+               "lsamp_test_rows_from_lists")
+    return np.array(out[:], bool)
+
+
 def draw_scale(cfg, r):
     """Draw scale of row r: fl(1/T) for mlx-lm sampled rows, else 1."""
     p = cfg["params"][r]

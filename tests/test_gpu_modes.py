@@ -85,10 +85,12 @@ def test_fused_equals_split_many_rounds(ctx):
 
 
 def test_fp32_steps_of_several_rounds_run_split(ctx):
-    """The fused kernel's several-rounds form is not built for the fp32 slab
-    (it would not fit the registers): such steps take the split kernels, in
-    every mode, with the same results."""
+    """The fused kernel's several-rounds form is not built for the fp32 slab (it
+    would not fit the registers): a batch past one round whose rows mostly
+    exchange histograms takes the split kernels, in every mode."""
     cfg = _many_rounds_cfg(_ffi.DTYPE_F32)
+    cfg["params"] = W._params([W.resolve_cbv2(temperature=[0.7, 1.0, 1.3][r % 3], top_k=[0, 400][r % 2],
+                                              vocab=cfg["vocab"]) for r in range(cfg["rows"])])
     f, s = _both_modes(ctx, cfg)
     _assert_same(f, s, "fp32 many rounds")
     for mode in (_ffi.MODE_AUTO, _ffi.MODE_FUSED):
@@ -98,6 +100,25 @@ def test_fp32_steps_of_several_rounds_run_split(ctx):
             assert ctx.last_launch()["fused"] == 0
         finally:
             ctx.set_mode(_ffi.MODE_AUTO)
+
+
+def test_fp32_list_rows_past_one_round_run_fused(ctx):
+    """Such a batch of argmax and top-k rows, which lists decide, takes the
+    fused kernel on a grid larger than the device (kind 5), with the split
+    kernels' results."""
+    cfg = _many_rounds_cfg(_ffi.DTYPE_F32)
+    cfg["params"] = W._params([W.resolve_cbv2(temperature=[0.0, 0.7, 1.0][r % 3], top_k=[40, 5, 90][r % 3],
+                                              top_p=[1.0, 0.9][r % 2], vocab=cfg["vocab"])
+                               for r in range(cfg["rows"])])
+    f, s = _both_modes(ctx, cfg)
+    _assert_same(f, s, "fp32 list rows past one round")
+    ctx.set_mode(_ffi.MODE_FUSED)
+    try:
+        run_gpu(ctx, cfg)
+        launch = ctx.last_launch()
+    finally:
+        ctx.set_mode(_ffi.MODE_AUTO)
+    assert launch["fused"] == 5 and launch["grid"] == cfg["rows"] * launch["slices"], launch
 
 
 def test_status_clear_after_default_mode(ctx):

@@ -10,7 +10,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from common import compare, run_gpu, run_oracle, to_torch_logits
+from common import compare, rows_from_lists, run_gpu, run_oracle, to_torch_logits
 from lsamp import _ffi
 from lsamp import workloads as W
 from lsamp.history import Cbv2RowState, TokenRing, csr, mlxlm_entries
@@ -84,12 +84,12 @@ def _batch(rows, V, dtype, sem, seed, masked):
 
 
 @pytest.mark.parametrize("rows,V,dtype,sem,masked", [
-    (200, 4099, _ffi.DTYPE_BF16, _ffi.SEM_CBV2, False),    # one slice a row
-    (120, 40003, _ffi.DTYPE_BF16, _ffi.SEM_MLXLM, False),  # two, unaligned rows
-    (80, 30720, _ffi.DTYPE_F16, _ffi.SEM_CBV2, True),      # three
+    (256, 4099, _ffi.DTYPE_BF16, _ffi.SEM_CBV2, False),    # one slice a row
+    (128, 40003, _ffi.DTYPE_BF16, _ffi.SEM_MLXLM, False),  # two, unaligned rows
+    (85, 9000, _ffi.DTYPE_F16, _ffi.SEM_CBV2, True),       # three
     (64, 65536, _ffi.DTYPE_F32, _ffi.SEM_CBV2, True),      # four
-    (60, 100000, _ffi.DTYPE_F32, _ffi.SEM_MLXLM, False),   # five: min-p alone
-    (20, 20480, _ffi.DTYPE_BF16, _ffi.SEM_CBV2, False),    # eight
+    (43, 9000, _ffi.DTYPE_F32, _ffi.SEM_MLXLM, False),     # five: min-p alone
+    (32, 65536, _ffi.DTYPE_BF16, _ffi.SEM_CBV2, False),    # eight: min-p alone
     (150, 70001, _ffi.DTYPE_F32, _ffi.SEM_CBV2, False),    # past one round
 ])
 def test_rows_from_lists(ctx, rows, V, dtype, sem, masked):
@@ -97,6 +97,12 @@ def test_rows_from_lists(ctx, rows, V, dtype, sem, masked):
     o = run_oracle(cfg, threads=16)
     lib = _ffi.load_library()
     compare(cfg, run_gpu(ctx, cfg), o, label="lists")
+    # rows of both outcomes; top-p rows go through lists of at most four slices
+    launch, lists = ctx.last_launch(), rows_from_lists(ctx, rows)
+    top_p = np.array([p["top_p"] < 1 for p in cfg["params"]])
+    assert lists[~top_p].any() and lists[top_p].any() == (launch["slices"] <= 4)
+    assert masked or not lists[6::10].any()  # (+inf logits, unless masked)
+    assert launch["fused"] == (5 if dtype == _ffi.DTYPE_F32 and rows == 150 else 1)
     ctx.read_status()
     _ffi.check(lib.lsamp_test_set_spin_limit(0, 16), "lsamp_test_set_spin_limit")
     try:

@@ -92,6 +92,7 @@ def test_fp32_batch_past_one_round_with_waits_given_up(ctx):
     o = run_oracle(cfg, threads=16)
     compare(cfg, _run_with_hook(ctx, cfg), o, label="hook on")
     compare(cfg, run_gpu(ctx, cfg), o, label="hook off")
+    assert ctx.last_launch()["fused"] == 5
     assert ctx.read_status() == 0
 
 
