@@ -50,6 +50,9 @@ using namespace dev;
 using namespace rowops;
 
 constexpr int kSpinLimit = 1 << 20;                   // ~0.2 s of polling
+// The anchors of the passes' mass sums are integers within this range (in log2
+// of mass); rows whose largest value lies outside take the histogram path.
+constexpr float kAnchorRange = 0x1p20f;
 // lsamp_test_set_spin_limit: > 0 makes every bounded wait's target unreachable and
 // its limit this many polls (the waits' fail-closed path, under test)
 __device__ int32_t g_spin_test = 0;
@@ -1746,7 +1749,7 @@ __device__ __forceinline__ void raw_add(RawAcc& a, uint4 v, uint32_t tail, uint3
   }
   a.m = __builtin_fmaxf(a.m, q);
   if (__builtin_fmaf(q, kLog2e, a.nb) > 64.0f) {
-    const float nn = -__builtin_ceilf(__builtin_amdgcn_fmed3f(q * kLog2e, -0x1p20f, 0x1p20f));
+    const float nn = -__builtin_ceilf(__builtin_amdgcn_fmed3f(q * kLog2e, -kAnchorRange, kAnchorRange));
     a.z = __builtin_ldexpf(a.z, (int)__builtin_fmaxf(nn - a.nb, -512.0f));
     a.nb = nn;
   }
@@ -2225,6 +2228,9 @@ __device__ __forceinline__ int find_count_bin(TaskLds& L, uint32_t need) {
 // sends the row down the histogram path, in the same launch, before the
 // exchange.
 constexpr int kNucP = 1, kNucM = 2;            // a row's filters: top-p, min-p
+// Values further than this below a maximum, in log2 of mass, weigh nothing
+// beside it (a slice's 65,536 of them 2^-48 of it, below a float's top-p step).
+constexpr float kNucRange = 64.0f;
 constexpr int kNucArea = kCandCap;             // keys of a row in each of two areas:
 static_assert(kMaxSlices * kKeptCap * sizeof(KeptItem) == kNucArea * sizeof(uint64_t),
               "cands and klist, both idle before the select phase");
@@ -2306,7 +2312,8 @@ __device__ __forceinline__ void nucleus_list(const Workspace& ws, const SamplePl
                                              int slice, const RowCtx& c,
                                              const lsamp_row_params& prm, int nuc, Slab<DT>& S,
                                              int nq, int32_t base32, int n_ent, float xmax,
-                                             float tmax, float tau, uint64_t ze, TaskLds& L,
+                                             float tmax, float tau, float low, uint64_t ze,
+                                             TaskLds& L,
                                              F&& qmax) {
   constexpr int N = Vec<DT>::N;
   const int tid = fresh_tid();
@@ -2343,6 +2350,7 @@ __device__ __forceinline__ void nucleus_list(const Workspace& ws, const SamplePl
       if (!(nuc & kNucP)) break;
       float unused;
       wave_reach(tmax, wave_max(tmax), nucleus_share(lay.seg, true) / 2, 1, tau, unused);
+      tau = __builtin_fmaxf(tau, low);
     }
     tcp = __builtin_fmaxf(__builtin_fmaxf(tau, tm), -__FLT_MAX__);
     // the quads that hold a listed token, staged whole
@@ -2970,9 +2978,9 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
       xmax = __builtin_elementwise_maximum(xmax, qm);
       if (zon) {
         // re-anchor when the quad's terms could pass 2^64 (an exact power-of-
-        // two rescale; the anchor is an integer, clamped to +-2^20)
+        // two rescale; the anchor is an integer, clamped to +-kAnchorRange)
         if (__builtin_fmaf(qm, lgz, nbz) > 64.0f) {
-          const float nn = -__builtin_ceilf(__builtin_amdgcn_fmed3f(qm * lgz, -0x1p20f, 0x1p20f));
+          const float nn = -__builtin_ceilf(__builtin_amdgcn_fmed3f(qm * lgz, -kAnchorRange, kAnchorRange));
           zt = __builtin_ldexpf(zt, (int)__builtin_fmaxf(nn - nbz, -512.0f));
           nbz = nn;
         }
@@ -3011,7 +3019,6 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
     // ------------------------------------------------ B: max
     if (nonfinite) atomicOr(&L.flags, LSAMP_ROW_NONFINITE);
     const float tmax = xmax;  // this thread's largest (transformed) logit
-    const float xthr = tmax;
     float tlo = kPosInf;      // smallest finite thread maximum (short lists, k > 1)
     // nucleus rows: the quads' maxima (16-bit types: kept in the area that the
     // list overwrites, so read into registers ahead of the barrier)
@@ -3031,6 +3038,9 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
       // how much mass lies below them in the whole slice.
       const int seg = nucleus_layout(G).seg;
       const float hi = wave_max(tmax);
+      // (maxima with next to no mass beside the wave's largest count as none:
+      // tokens filled with a very low finite value)
+      const float vmax = tmax > hi - kNucRange / lgz ? tmax : kNegInf;
       float q_few = kNegInf, q_many = kNegInf;
       double zsum = 0.0;
       float z_few = 0.0f, z_many = 0.0f;
@@ -3042,10 +3052,14 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
         const float bh = hi * lgz;
         const float bl = __builtin_fmaf(hi, lgz, -bh);
         const float dl = tmax > kNegInf ? (tmax - hi) * lgl : 0.0f;
-        const float zr = zref ? zt * __builtin_amdgcn_exp2f(((-nbz - bh) - bl) + dl) : 0.0f;
+        // (a wave below the anchors' range has no sum: the slice's range
+        // check, below, or the slice's larger tokens make it irrelevant)
+        const float zr = zref && bh > -kAnchorRange
+                             ? zt * __builtin_amdgcn_exp2f(((-nbz - bh) - bl) + dl)
+                             : 0.0f;
         zsum = wave_sum((double)zr);
         if ((nuc & kNucP) != 0) {
-          wave_reach(tmax, hi, nucleus_share(seg, true), nucleus_share(seg, false), q_few, q_many);
+          wave_reach(vmax, hi, nucleus_share(seg, true), nucleus_share(seg, false), q_few, q_many);
           const bool bf = tmax < q_few, bm = tmax < q_many;
           z_few = wave_sum(bf ? zr : 0.0f);
           z_many = wave_sum(bm ? zr : 0.0f);
@@ -3122,7 +3136,8 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
       uint32_t* const sync = row_sync(ws, row);
       const int wv = tid >> 6;
       // (no list: +inf logits, an entry-table overflow, a sum out of range)
-      const bool bad = posinf || ent_overflow || (zon && has_finite && !(xmax * lgz < 0x1p20f));
+      const bool bad = posinf || ent_overflow ||
+                       (zon && has_finite && !(__builtin_fabsf(xmax * lgz) < kAnchorRange));
       if (tid == 0) {
         st_coherent_f32(&Ssum->x_max, xmax);
         st_coherent(&Ssum->top_bin, top);
@@ -3155,8 +3170,10 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
         // The list's size (entries apart): few when the mass below their
         // threshold is well below what top-p drops, else many, unless even
         // theirs leaves out more than top-p drops.  The thresholds are the
-        // waves' averaged (a wave with too few finite maxima lists all it has).
-        float tau = kNegInf;
+        // waves' averaged (a wave with too few maxima lists all it has down to
+        // `low`), waves far below the slice's maximum apart.
+        const float low = (nuc & kNucP) != 0 ? xmax - kNucRange / lgz : kNegInf;
+        float tau = low;
         if ((nuc & kNucP) != 0) {
           // (over 8 lanes: two quad permutes and a half-row mirror)
           auto sum8 = [](float v) {
@@ -3173,16 +3190,17 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
           const bool is_few = u_few <= 0.7f * drop * s_few;
           wide = !is_few && u_many > 0.85f * drop * s_many;
           const float qw = is_few ? nw.q_few : nw.q_many;
-          const float sum = sum8(qw > kNegInf ? qw : 0.0f);
-          const float cnt = sum8(qw > kNegInf ? 1.0f : 0.0f);
-          if (read_lane(qw, wv) > kNegInf)
+          const bool near = qw > kNegInf && nw.hi > low;
+          const float sum = sum8(near ? qw : 0.0f);
+          const float cnt = sum8(near ? 1.0f : 0.0f);
+          if (read_lane(qw, wv) > kNegInf && read_lane(cnt, 0) > 0.0f)
             tau = __uint_as_float(
                 (uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(sum / cnt)));
         }
         wide = __builtin_amdgcn_readfirstlane(wide ? 1 : 0) != 0;
         if (!wide)
-          nucleus_list<DT>(ws, P, row, slice, c, prm, nuc, S, nq, base32, n_ent, xmax, xthr, tau,
-                           ze, L, qmax);
+          nucleus_list<DT>(ws, P, row, slice, c, prm, nuc, S, nq, base32, n_ent, xmax,
+                           tmax > low ? tmax : kNegInf, tau, low, ze, L, qmax);
       } else if (!bad && (tid & 63) == 0) {
         // (nothing finite)
         st_coherent(&Ssum->part[wv], (uint64_t)0xff800000u << 32);
@@ -3293,7 +3311,8 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
         // rounding error (exact through an fma) is common to them all
         const float nb = -xmax * lgz;
         const float nb_err = __builtin_fmaf(-xmax, lgz, -nb);
-        if (zon && !(xmax * lgz < 0x1p20f)) sflags |= kSliceShortOverflow;  // out of range
+        if (zon && !(__builtin_fabsf(xmax * lgz) < kAnchorRange))
+          sflags |= kSliceShortOverflow;  // out of range
         // candidates are the tokens x >= tcp (tcp >= -FLT_MAX also rules out
         // -inf).  A quad holding one is staged whole in the thread's next LDS
         // slot (past kQStage into a discard slot) and its candidates counted,

@@ -143,3 +143,66 @@ def test_rows_without_filters(ctx, rows, V, dtype):
         assert np.array_equal(out["tokens"].cpu().numpy(), full["tokens"])
         assert np.array_equal(out["row_flags"].cpu().numpy().astype(np.uint32), full["row_flags"])
     assert ctx.read_status() == 0
+
+
+def _sparse(V, ids, values):
+    x = np.full(V, -np.inf)
+    x[ids] = values
+    return x
+
+
+@pytest.mark.parametrize("rows,V,dtype", [
+    (64, 65536, _ffi.DTYPE_F32), (64, 65536, _ffi.DTYPE_F16), (43, 9000, _ffi.DTYPE_F32),
+    (256, 4099, _ffi.DTYPE_BF16)])
+@pytest.mark.parametrize("sem", [_ffi.SEM_CBV2, _ffi.SEM_MLXLM])
+def test_values_far_from_zero(ctx, rows, V, dtype, sem):
+    """Rows whose surviving logits lie beyond the range in which a slice sums its
+    mass (|x| / T past 2^20 log2 units; temperatures that divide such values
+    exactly), and ordinary rows beside tokens filled with a very low finite
+    value: some tokens, whole waves or whole slices."""
+    rng = np.random.default_rng(V + dtype)
+    x = rng.normal(0, 3, (rows, V))
+    # (bins of 1/32 stay exact in float32 up to 2^19)
+    far = 6e4 if dtype == _ffi.DTYPE_F16 else 2.5e5
+    fill = {_ffi.DTYPE_F16: -65504.0, _ffi.DTYPE_BF16: -3.3895e38}.get(dtype, -3.4028235e38)
+    T = np.full(rows, 0.8)
+    for r in range(rows):
+        kind, ids = r % 8, rng.choice(V, 3, replace=False)
+        if kind == 0:  # three equal tokens far below
+            x[r] = _sparse(V, ids, -far)
+        elif kind == 1:  # and far above
+            x[r] = _sparse(V, ids, far)
+        elif kind == 2:  # a few hundred steps of the type's own spacing, far below
+            ids = rng.choice(V, 300, replace=False)
+            x[r] = _sparse(V, ids, -far + 0.0625 * rng.integers(0, 200, 300))
+        elif kind == 3:  # most tokens filled low
+            x[r, rng.random(V) < 0.97] = -1e9 if dtype != _ffi.DTYPE_F16 else fill
+        elif kind == 4:  # a slice and more of them
+            x[r, : V // 3] = fill
+        elif kind == 5:  # every token but a few hundred
+            keep = rng.choice(V, 300, replace=False)
+            x[r] = np.where(np.isin(np.arange(V), keep), x[r], fill)
+        elif kind == 6:  # the largest value far below, a cold row
+            ids = rng.choice(V, 300, replace=False)
+            x[r] = _sparse(V, ids, rng.normal(-3e4, 3, 300))
+            T[r] = 2.0 ** -5
+        if kind < 3:
+            T[r] = 2.0 ** -5 if dtype == _ffi.DTYPE_F16 else 0.25
+    params = []
+    for r in range(rows):
+        kw = dict(temperature=float(T[r]), top_p=[0.9, 0.97, 1.0][r // 8 % 3],
+                  min_p=[0.0, 0.02, 0.05][r // 8 % 3])
+        params.append(W.resolve_cbv2(vocab=V, **kw) if sem == _ffi.SEM_CBV2 else
+                      W.resolve_mlxlm(**kw))
+    with np.errstate(over="ignore"):
+        cfg = dict(semantics=sem, dtype=dtype, rows=rows, vocab=V, logits=_bits(x, dtype),
+                   params=W._params(params), row_ptr=None, entries=None, bitmask=None, mask_bits=0,
+                   uniforms=rng.random(rows, dtype=np.float32))
+    o = run_oracle(cfg, threads=16)
+    g = run_gpu(ctx, cfg)
+    compare(cfg, g, o, label="far")
+    fin = np.isfinite(o["stats"]["log_normalizer"])
+    gn, on = g["stats"]["log_normalizer"][fin], o["stats"]["log_normalizer"][fin]
+    bad = np.abs(gn - on) > 2e-6 * (1 + np.abs(on))
+    assert not bad.any(), (np.nonzero(fin)[0][bad], gn[bad], on[bad])
+    assert ctx.read_status() == 0
