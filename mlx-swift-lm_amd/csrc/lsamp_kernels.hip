@@ -2949,7 +2949,13 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
   float xmax = kNegInf;
   // exp-sum anchor: nbz starts above every quad, so the first finite quad
   // anchors, and the shift of that first anchor clears what came before
-  float zt = 0.0f, nbz = __FLT_MAX__;
+  float nbz = __FLT_MAX__;
+  // (a quad's terms are added among themselves, a bank's quads in fp32, the
+  // banks in double: one running fp32 sum lost up to 127 terms of just under
+  // 2^-25 after a dominant one, 3.8e-6 of the mass, where top-p's boundary is
+  // held to 1e-6; now 7 quads' at most, 4e-7)
+  double zt = 0.0;
+  float zb = 0.0f;
   // (LP, own pass) the raw logits' statistics, before any exclusion
   RawAcc ra{kNegInf, 0.0f, __FLT_MAX__, 0u};
   auto first_pass = [&](int g, uint4& v) {
@@ -2981,12 +2987,20 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
         // two rescale; the anchor is an integer, clamped to +-kAnchorRange)
         if (__builtin_fmaf(qm, lgz, nbz) > 64.0f) {
           const float nn = -__builtin_ceilf(__builtin_amdgcn_fmed3f(qm * lgz, -kAnchorRange, kAnchorRange));
-          zt = __builtin_ldexpf(zt, (int)__builtin_fmaxf(nn - nbz, -512.0f));
+          const int by = (int)__builtin_fmaxf(nn - nbz, -512.0f);
+          zt = __builtin_ldexp(zt, by);
+          zb = __builtin_ldexpf(zb, by);
           nbz = nn;
         }
+        float t[N];
 #pragma unroll
         for (int e = 0; e < N; ++e)
-          zt += __builtin_amdgcn_exp2f(__builtin_fmaf(vec_elem<DT>(v, e), lgz, nbz));
+          t[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(vec_elem<DT>(v, e), lgz, nbz));
+#pragma unroll
+        for (int w = 1; w < N; w *= 2)
+#pragma unroll
+          for (int e = 0; e < N; e += 2 * w) t[e] += t[e + w];
+        zb += t[0];
       }
     }
   };
@@ -3002,6 +3016,8 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
         quad_set(S.bank[b], s, v);
       }
     }
+    zt += (double)zb;
+    zb = 0.0f;
   }
   const bool zref = nbz < __FLT_MAX__;
   finish_slice_entries<DT>(P, c, prm, mrow, se, ep, em, emax);
@@ -3054,15 +3070,15 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
         const float dl = tmax > kNegInf ? (tmax - hi) * lgl : 0.0f;
         // (a wave below the anchors' range has no sum: the slice's range
         // check, below, or the slice's larger tokens make it irrelevant)
-        const float zr = zref && bh > -kAnchorRange
-                             ? zt * __builtin_amdgcn_exp2f(((-nbz - bh) - bl) + dl)
-                             : 0.0f;
-        zsum = wave_sum((double)zr);
+        const double zr = zref && bh > -kAnchorRange
+                              ? zt * (double)__builtin_amdgcn_exp2f(((-nbz - bh) - bl) + dl)
+                              : 0.0;
+        zsum = wave_sum(zr);
         if ((nuc & kNucP) != 0) {
           wave_reach(vmax, hi, nucleus_share(seg, true), nucleus_share(seg, false), q_few, q_many);
           const bool bf = tmax < q_few, bm = tmax < q_many;
-          z_few = wave_sum(bf ? zr : 0.0f);
-          z_many = wave_sum(bm ? zr : 0.0f);
+          z_few = wave_sum(bf ? (float)zr : 0.0f);
+          z_many = wave_sum(bm ? (float)zr : 0.0f);
           n_few = (int)__popcll(__ballot(bf));
           n_many = (int)__popcll(__ballot(bm));
         }
@@ -3364,9 +3380,10 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
         // (xmax * lgz split into a rounded part and its exact residual)
         const float bh = xmax * lgz;
         const float bl = __builtin_fmaf(xmax, lgz, -bh);
-        const float zr = (zon && zref) ? zt * __builtin_amdgcn_exp2f((-nbz - bh) - bl) : 0.0f;
+        const double zr =
+            (zon && zref) ? zt * (double)__builtin_amdgcn_exp2f((-nbz - bh) - bl) : 0.0;
         // (each term is at most 1, so zr <= 128; out-of-range rows fall back)
-        ze += zr < 0x1p20f ? (uint64_t)(zr * 0x1p40f) : 0ull;
+        ze += zr < 0x1p20 ? (uint64_t)(zr * 0x1p40) : 0ull;
         ze = wave_sum(ze);
         const int wv = tid >> 6;
         __syncthreads();

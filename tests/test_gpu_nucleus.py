@@ -206,3 +206,37 @@ def test_values_far_from_zero(ctx, rows, V, dtype, sem):
     bad = np.abs(gn - on) > 2e-6 * (1 + np.abs(on))
     assert not bad.any(), (np.nonzero(fin)[0][bad], gn[bad], on[bad])
     assert ctx.read_status() == 0
+
+
+@pytest.mark.parametrize("dtype", [_ffi.DTYPE_F32, _ffi.DTYPE_BF16])
+@pytest.mark.parametrize("first", [True, False])
+def test_mass_of_a_dominant_token_and_its_thread(ctx, dtype, first):
+    """One token ahead of the 127 others of its thread, each just under 2^-25 of
+    its mass (3.8e-6 together), and a rest that weighs nothing: top-p cuts inside
+    the 127, where the row's mass decides how many stay (a running fp32 sum kept
+    the dominant token alone).  Statistics against 64 bits."""
+    rows, V = 256, 65536
+    N = 4 if dtype == _ffi.DTYPE_F32 else 8
+    rng = np.random.default_rng(dtype + first)
+    x = rng.normal(-30, 1, (rows, V))
+    mine = (np.arange(128) // N) * 512 * N + np.arange(128) % N  # thread 0 of a whole slice
+    for r in range(rows):
+        ids = mine + N * (r % 512)
+        # 2^-25 is 17.33 nats; bf16 steps there are 1/8
+        x[r, ids] = -(17.34 + 1e-3 * rng.random(128)) if N == 4 else -17.375
+        x[r, ids[0 if first else 127]] = 0.0
+    top_p = [np.float32(1) - np.float32(k * 2.0 ** -24) for k in (26, 30, 34, 38)]
+    params = [W.resolve_cbv2(temperature=1.0, top_p=float(top_p[r % 4]), vocab=V)
+              for r in range(rows)]
+    cfg = dict(semantics=_ffi.SEM_CBV2, dtype=dtype, rows=rows, vocab=V, logits=_bits(x, dtype),
+               params=W._params(params), row_ptr=None, entries=None, bitmask=None, mask_bits=0,
+               uniforms=rng.random(rows, dtype=np.float32))
+    o = run_oracle(cfg, threads=16)
+    g = run_gpu(ctx, cfg)
+    assert ctx.last_launch()["slices"] == 1 and rows_from_lists(ctx, rows).all()
+    compare(cfg, g, o, label="dominant")
+    assert (g["stats"]["kept"] > 16).all()
+    y = W.bf16_bits_to_f32(cfg["logits"]) if N == 8 else cfg["logits"]
+    z = np.log(np.exp(y.astype(np.float64)).sum(1))
+    # (3.8e-6 of the mass in all; the sum's own error is below a tenth of it)
+    assert np.abs(g["stats"]["log_normalizer"] - z).max() < 5e-7
