@@ -763,6 +763,64 @@ __device__ __forceinline__ void write_row(const Workspace& ws, const SamplePlan&
   ws.rows[row] = out;
 }
 
+// Sorts F.keys[0 .. nc), nc >= 2, in descending order (keys are distinct: ids
+// are).  Whole work-group, the keys complete; ends in a barrier.
+__device__ __forceinline__ void sort_keys(TaskLds& L, int nc) {
+  const int tid = fresh_tid();
+  FinalLds& F = L.u.f;
+  if (nc <= kThreads) {
+    // rank by counting, spread over the work-group: thread (i, ch) counts the
+    // keys above key i in chunk ch of the list (kThreads over nc rounded up to
+    // a power of two chunks; 125 keys: 2.3 us with a thread per key)
+    uint32_t* const above = L.sh.tcnt;
+    static_assert(kTauBins >= kThreads, "a count per candidate");
+    const uint64_t own = tid < nc ? F.keys[tid] : 0ull;
+    above[tid] = 0u;
+    __syncthreads();
+    const int np = nc <= 64 ? 64 : nc <= 128 ? 128 : nc <= 256 ? 256 : 512;
+    const int i = tid & (np - 1), span = (nc * np + kThreads - 1) / kThreads;
+    const int j0 = tid / np * span, j1 = j0 + span < nc ? j0 + span : nc;
+    if (i < nc) {
+      const uint64_t key = F.keys[i];
+      int r = 0;
+      int j = j0;
+      for (; j + 8 <= j1; j += 8) {  // (eight reads in flight)
+        uint64_t k8[8];
+#pragma unroll
+        for (int d = 0; d < 8; ++d) k8[d] = F.keys[j + d];
+#pragma unroll
+        for (int d = 0; d < 8; ++d) r = add_gt_u64(r, k8[d], key);
+      }
+      for (; j < j1; ++j) r = add_gt_u64(r, F.keys[j], key);
+      if (r != 0) atomicAdd(&above[i], (uint32_t)r);
+    }
+    __syncthreads();
+    if (tid < nc) F.keys[above[tid]] = own;
+    __syncthreads();
+    return;
+  }
+  int n2 = 1;
+  while (n2 < nc) n2 <<= 1;
+  for (int i = nc + tid; i < n2; i += kThreads) F.keys[i] = 0ull;
+  __syncthreads();
+  for (int kk = 2; kk <= n2; kk <<= 1) {
+    for (int jj = kk >> 1; jj > 0; jj >>= 1) {
+      for (int i = tid; i < n2; i += kThreads) {
+        const int ixj = i ^ jj;
+        if (ixj > i) {
+          const uint64_t a = F.keys[i], b = F.keys[ixj];
+          const bool desc = (i & kk) == 0;
+          if (desc ? (a < b) : (a > b)) {
+            F.keys[i] = b;
+            F.keys[ixj] = a;
+          }
+        }
+      }
+      __syncthreads();
+    }
+  }
+}
+
 // The keep rule over a row's sorted cut-bin candidates in F.keys (one wave,
 // 64 at a time): the kept ones' weights go to F.rowchunk, F.keep marks them,
 // and they are listed in ws.cands.
@@ -1191,64 +1249,17 @@ __device__ __forceinline__ void finalize_row(const Workspace& ws, const SamplePl
   nc = L.misc[1];
 
   // ---- sort candidates: value descending, id ascending (-0 == +0)
-  if (nc > 64 && nc <= kThreads) {
-    // rank by counting (keys are distinct: ids are), spread over the work-
-    // group: thread (i, ch) counts the keys above key i in chunk ch of the
-    // list (kThreads over nc rounded up to a power of two chunks; 125 keys:
-    // 2.3 us with a thread per key)
-    uint32_t* const above = L.sh.tcnt;
-    static_assert(kTauBins >= kThreads, "a count per candidate");
-    if (tid < nc) F.dw[tid] = key0;
-    above[tid] = 0u;
-    __syncthreads();
-    const int np = nc <= 128 ? 128 : nc <= 256 ? 256 : 512;
-    const int i = tid & (np - 1), span = (nc * np + kThreads - 1) / kThreads;
-    const int j0 = tid / np * span, j1 = j0 + span < nc ? j0 + span : nc;
-    if (i < nc) {
-      const uint64_t key = F.dw[i];
-      int r = 0;
-      int j = j0;
-      for (; j + 8 <= j1; j += 8) {  // (eight reads in flight)
-        uint64_t k8[8];
-#pragma unroll
-        for (int d = 0; d < 8; ++d) k8[d] = F.dw[j + d];
-#pragma unroll
-        for (int d = 0; d < 8; ++d) r = add_gt_u64(r, k8[d], key);
-      }
-      for (; j < j1; ++j) r = add_gt_u64(r, F.dw[j], key);
-      if (r != 0) atomicAdd(&above[i], (uint32_t)r);
-    }
-    __syncthreads();
-    if (tid < nc) F.keys[above[tid]] = key0;
-    __syncthreads();
-  } else if (nc > 64) {
-    int n2 = 1;
-    while (n2 < nc) n2 <<= 1;
-    for (int i = tid; i < n2; i += kThreads) {
-      uint64_t key = 0ull;
-      if (i < nc) {
+  if (nc > 64) {
+    if (nc <= kThreads) {
+      if (tid < nc) F.keys[tid] = key0;
+    } else {
+      for (int i = tid; i < nc; i += kThreads) {
         const float y = __uint_as_float(ld_coherent(reinterpret_cast<const uint32_t*>(&rc[i].y)));
-        key = cand_key(y, ld_coherent(&rc[i].id));
+        F.keys[i] = cand_key(y, ld_coherent(&rc[i].id));
       }
-      F.keys[i] = key;
     }
     __syncthreads();
-    for (int kk = 2; kk <= n2; kk <<= 1) {
-      for (int jj = kk >> 1; jj > 0; jj >>= 1) {
-        for (int i = tid; i < n2; i += kThreads) {
-          const int ixj = i ^ jj;
-          if (ixj > i) {
-            const uint64_t a = F.keys[i], b = F.keys[ixj];
-            const bool desc = (i & kk) == 0;
-            if (desc ? (a < b) : (a > b)) {
-              F.keys[i] = b;
-              F.keys[ixj] = a;
-            }
-          }
-        }
-        __syncthreads();
-      }
-    }
+    sort_keys(L, nc);
   }
   if (!wave0) {
     // (wave 1: the raw log-probability lists, beside wave 0's draw, in the
@@ -2664,25 +2675,7 @@ __device__ __forceinline__ bool nucleus_row(const Workspace& ws, const SamplePla
   __syncthreads();
   const bool overflow = L.ncand > kCandCap;
   const int nc = overflow || !active ? 0 : L.ncand;
-  // the cut bin's keys ranked by counting (keys are distinct: ids are)
-  if (nc > 1) {
-    constexpr int kPer = kCandCap / kThreads;
-    uint64_t key[kPer];
-    int r[kPer];
-#pragma unroll
-    for (int k = 0; k < kPer; ++k) {
-      const int i = tid + k * kThreads;
-      key[k] = i < nc ? F.keys[i] : 0ull;
-      r[k] = 0;
-      if (k * kThreads < nc && i < nc)
-        for (int j = 0; j < nc; ++j) r[k] = add_gt_u64(r[k], F.keys[j], key[k]);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < kPer; ++k)
-      if (tid + k * kThreads < nc) F.keys[r[k]] = key[k];
-    __syncthreads();
-  }
+  if (nc > 1) sort_keys(L, nc);
   const bool draw = !P.bonus_only || (row < P.rows_split && row % P.vwin == P.vwin - 1);
   KeptCands kc{0, 0.0, kPosInf};
   uint64_t W = 0ull;

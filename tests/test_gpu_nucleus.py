@@ -240,3 +240,26 @@ def test_mass_of_a_dominant_token_and_its_thread(ctx, dtype, first):
     z = np.log(np.exp(y.astype(np.float64)).sum(1))
     # (3.8e-6 of the mass in all; the sum's own error is below a tenth of it)
     assert np.abs(g["stats"]["log_normalizer"] - z).max() < 5e-7
+
+
+@pytest.mark.parametrize("n", [12, 63, 65, 127, 300, 511, 513, 1025, 1800])
+def test_ties_in_the_cut_bin(ctx, n):
+    """Nuclei that end inside n equal tokens: the cut bin's keys are ranked by
+    counting up to a work-group's threads and sorted past that."""
+    rows, V = 64, 65536
+    rng = np.random.default_rng(n)
+    x = rng.normal(-12, 0.5, (rows, V))
+    for r in range(rows):
+        # (some in each of the row's four slices, so that no slice is flat)
+        ids = rng.choice(V // 4, n + 1, replace=False) + V // 4 * (np.arange(n + 1) % 4)
+        x[r, ids] = 2.0
+        x[r, ids[0]] = 2.0 + [0.0, 1.5][r % 2]
+    top_p = [0.3, 0.9, 0.97, 0.6]
+    params = [W.resolve_cbv2(temperature=0.7, top_p=top_p[r % 4], vocab=V) for r in range(rows)]
+    cfg = dict(semantics=_ffi.SEM_CBV2, dtype=_ffi.DTYPE_F16, rows=rows, vocab=V,
+               logits=_bits(x, _ffi.DTYPE_F16), params=W._params(params), row_ptr=None, entries=None,
+               bitmask=None, mask_bits=0, uniforms=rng.random(rows, dtype=np.float32))
+    o = run_oracle(cfg, threads=16)
+    g = run_gpu(ctx, cfg)
+    assert rows_from_lists(ctx, rows).all()
+    compare(cfg, g, o, label=f"{n} ties")
