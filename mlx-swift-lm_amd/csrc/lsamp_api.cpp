@@ -154,6 +154,32 @@ void plan_slices(int32_t rows, int32_t vocab, int32_t slots, int32_t* slices, in
   *nchunks = nch;
 }
 
+// An fp32 batch past one round of `slots` work-groups (the several-rounds form
+// is not built for the fp32 slab: it would not fit the registers): as few
+// launches of the one-round kernel as the longest slices allow, the rows spread
+// evenly over them, each on a grid that fits the device at once.  Returns the
+// rows of a launch, or 0, the plan as it was, where several launches would leave
+// more than a sixteenth of their slots idle: the split kernels' grid has no such
+// gaps (verification, 224 rows x 151,936 in three launches of 75, 433 us, split
+// 396; 128 x 100,000 in one launch 40, split 44).  (One launch over a larger grid
+// starts a row's slices apart, and the last one did the others' selects:
+// 128 rows x 151,936 verified without filters 397 us, the split kernels 252.)
+int32_t plan_launches(int32_t rows, int32_t vocab, int32_t slots, int32_t* slices,
+                      int32_t* slice_len, int32_t* nchunks) {
+  const int32_t g_min = (vocab + kMaxSliceLen - 1) / kMaxSliceLen;
+  const int32_t most = slots / g_min;  // rows a launch holds
+  const int32_t launches = (rows + most - 1) / most;
+  const int32_t per = (rows + launches - 1) / launches;
+  int32_t g = 0, len = 0, nch = 0;
+  // (as many slots as whole slices of those rows fill)
+  plan_slices(per, vocab, slots / per * per, &g, &len, &nch);
+  if (launches > 1 && 16 * (int64_t)rows * g < 15 * (int64_t)launches * slots) return 0;
+  *slices = g;
+  *slice_len = len;
+  *nchunks = nch;
+  return per;
+}
+
 // Rows of top-p / min-p alone go through lists in the one-round kernel.  Where
 // a work-group takes several tasks (16-bit batches past one round) a row's
 // histograms cost about what its lists and their wait do, and a row wider than
@@ -314,22 +340,30 @@ lsamp_status lsamp::sample_step(const WorkspaceViews& v, const DeviceShape& d, i
   // (the top-k kernel: one work-group per CU is enough, and fewer slices per
   // row mean a shorter merge)
   plan_slices(a->rows, a->vocab, topk ? d.cus : slots, &P.slices, &P.slice_len, &P.nchunks);
-  // An fp32 batch past one round of the grid (the several-rounds form is not
-  // built for the fp32 slab: it would not fit the registers) runs the one-round
-  // kernel over a grid larger than the device: its hand-off assumes no
-  // co-residency, so the dispatcher's own order serves.  128 rows x 151,936
-  // with top-p: 71 us, the split kernels (which read every slice twice) 101.
-  // A batch most of whose rows exchange histograms keeps the split kernels
-  // (193 rows x 32,000 without filters: 131 us, 161 in one kernel, whose
-  // slices wait for each other), and so does one that asks for raw
+  // An fp32 batch past one round of the grid: launches of one round each, where
+  // at least half of its rows are drawn from lists (128 rows x 151,936 with
+  // top-p: 75 us, the split kernels, which read every slice twice, 101).  Others
+  // keep the split kernels, and so does a batch that asks for raw
   // log-probabilities.
-  const bool over = a->dtype == LSAMP_DTYPE_F32 && (int64_t)a->rows * P.slices > slots;
-  const RowMix mix = row_mix(a, P.slices);
-  P.fused = !topk && mode != LSAMP_MODE_SPLIT && bpc > 0 && slots >= P.slices &&
-            (!over || (mix.lists && !(lp && lp->k >= 0)));
-  P.rows_per_round = P.fused && !over ? slots / P.slices : a->rows;
-  if (!topk && mix.nucleus)
-    P.fused |= nucleus_lists(a->dtype, (int64_t)a->rows * P.slices, slots);
+  bool one = !topk && bpc > 0 && slots >= P.slices;
+  const bool over = one && a->dtype == LSAMP_DTYPE_F32 && (int64_t)a->rows * P.slices > slots;
+  int32_t per = slots / P.slices;
+  RowMix mix = topk ? RowMix{false, false} : row_mix(a, P.slices);
+  if (over) {
+    int32_t slices = P.slices, slice_len = P.slice_len;
+    per = lp && lp->k >= 0 ? 0
+                           : plan_launches(a->rows, a->vocab, slots, &slices, &slice_len, &P.nchunks);
+    const RowMix there = per > 0 ? row_mix(a, slices) : RowMix{false, false};
+    one = there.lists;
+    if (one) {  // (also in split mode: the same slices)
+      mix = there;
+      P.slices = slices;
+      P.slice_len = slice_len;
+    }
+  }
+  P.fused = one && mode != LSAMP_MODE_SPLIT;
+  P.rows_per_round = P.fused ? per : a->rows;
+  if (mix.nucleus) P.fused |= nucleus_lists(a->dtype, (int64_t)a->rows * P.slices, slots);
   const size_t es = a->dtype == LSAMP_DTYPE_F32 ? 4 : 2;
   P.aligned = aligned16(a->logits) && ((size_t)a->row_stride * es) % 16 == 0;
   P.logits = a->logits;
@@ -390,11 +424,11 @@ lsamp_status lsamp::sample_step(const WorkspaceViews& v, const DeviceShape& d, i
     flp.ids = lp->ids;
     flp.rec = v.rawrec;
   }
-  last->fused = topk                          ? (lp_fused ? 3 : 2)
-                : lp_sample                   ? 4
-                : !(P.fused & kPlanFused)     ? 0
-                : over                        ? 5
-                                              : 1;
+  last->fused = topk                                    ? (lp_fused ? 3 : 2)
+                : lp_sample                             ? 4
+                : !(P.fused & kPlanFused)               ? 0
+                : over && P.rows > P.rows_per_round     ? 5
+                                                        : 1;
   last->slices = P.slices;
   last->slice_len = P.slice_len;
   last->rows_per_round = P.rows_per_round;
@@ -1076,10 +1110,15 @@ lsamp_status lsamp_verify(lsamp_context* ctx, const lsamp_verify_args* a, void* 
   const int32_t bpc = ctx->shape.fused_bpc[a->dtype];
   const int32_t slots = ctx->cus * (bpc > 0 ? bpc : 1);
   plan_slices(P.rows, P.vocab, slots, &P.slices, &P.slice_len, &P.nchunks);
-  // (fp32 rows past one round: as in sample_step)
-  P.fused = ctx->mode != LSAMP_MODE_SPLIT && bpc > 0 && slots >= P.slices;
-  const bool over = a->dtype == LSAMP_DTYPE_F32 && (int64_t)P.rows * P.slices > slots;
-  P.rows_per_round = P.fused && !over ? slots / P.slices : P.rows;
+  bool one = bpc > 0 && slots >= P.slices;
+  int32_t per = slots / P.slices;
+  // (fp32 past one round; nothing is known of the rows here)
+  if (one && a->dtype == LSAMP_DTYPE_F32 && (int64_t)P.rows * P.slices > slots) {
+    per = plan_launches(P.rows, P.vocab, slots, &P.slices, &P.slice_len, &P.nchunks);
+    one = per > 0;
+  }
+  P.fused = one && ctx->mode != LSAMP_MODE_SPLIT;
+  P.rows_per_round = P.fused ? per : P.rows;
   P.fused |= nucleus_lists(a->dtype, (int64_t)P.rows * P.slices, slots);
   const size_t es = a->dtype == LSAMP_DTYPE_F32 ? 4 : 2;
   P.aligned = aligned16(a->target_logits) && (!residual || aligned16(a->draft_logits)) &&

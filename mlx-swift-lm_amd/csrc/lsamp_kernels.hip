@@ -3947,8 +3947,8 @@ __device__ __forceinline__ uint32_t run_task(const Workspace& ws, const SamplePl
 
 // ================================================================ kernels
 // ONE: a work-group per task (no loop over rounds, so nothing is hoisted out
-// of one and spilled before the first load): every row fits one round of the
-// grid, or (fp32) the grid is larger than the device.
+// of one and spilled before the first load): every row of the launch, from
+// row0 on, fits one round of the grid.
 // NUC (with ONE): nucleus rows go through lists.  A batch whose host copy of the
 // parameters shows no such row runs the kernel without that code, which costs
 // the other rows 0.5 to 1.5 us by its registers and its size.
@@ -3966,9 +3966,10 @@ __global__ __launch_bounds__(kThreads) void k_fused(Workspace wsk, SamplePlan Pk
   const int rowslot = (int)blockIdx.x / G;
   const int slice = (int)blockIdx.x % G;
   if (ONE) {
-    if (rowslot < P.rows) {
-      const uint32_t out = run_task<DT, kFused, LP, NUC>(ws, P, rowslot, slice, L, Lk);
-      if (threadIdx.x == 0) clear_if_last(ws, rowslot, G, out);
+    const int row = P.row0 + rowslot;
+    if (row < P.rows) {
+      const uint32_t out = run_task<DT, kFused, LP, NUC>(ws, P, row, slice, L, Lk);
+      if (threadIdx.x == 0) clear_if_last(ws, row, G, out);
     }
     return;
   }
@@ -4069,22 +4070,26 @@ int launch_dt(const Workspace& ws, const SamplePlan& P, const FusedLp* lp, hipSt
   };
   mark(0);
   if (P.fused & kPlanFused) {
-    const int rounds_rows = P.rows < P.rows_per_round ? P.rows : P.rows_per_round;
-    const dim3 grid((unsigned)(rounds_rows * P.slices));
     const FusedLp none{-1, nullptr, nullptr, nullptr, nullptr};
     const FusedLp& lk = lp ? *lp : none;
-    // (fp32 steps have no several-rounds instantiation: with the fp32 slab it
-    // does not fit the registers.  The planner gives a batch past one round a
-    // grid of one work-group per task, which the dispatcher starts in order as
-    // work-groups end)
     const bool nuc = (P.fused & kPlanLists) != 0;
     auto kf = lp ? (nuc ? k_fused<DT, true, true, true> : k_fused<DT, true, true, false>)
                  : (nuc ? k_fused<DT, true, false, true> : k_fused<DT, true, false, false>);
-    if constexpr (DT != LSAMP_DTYPE_F32) {
+    auto launch = [&](const SamplePlan& Pl, int rows) {
+      hipLaunchKernelGGL(kf, dim3((unsigned)(rows * P.slices)), dim3(kThreads), 0, st, ws, Pl, lk);
+    };
+    const int per = P.rows < P.rows_per_round ? P.rows : P.rows_per_round;
+    // (fp32 steps have no several-rounds instantiation: with the fp32 slab it
+    // does not fit the registers)
+    if constexpr (DT == LSAMP_DTYPE_F32) {
+      SamplePlan Pl = P;
+      for (Pl.row0 = 0; Pl.row0 < P.rows; Pl.row0 += per)
+        launch(Pl, P.rows - Pl.row0 < per ? P.rows - Pl.row0 : per);
+    } else {
       if (P.rows > P.rows_per_round)
         kf = lp ? k_fused<DT, false, true, false> : k_fused<DT, false, false, false>;
+      launch(P, per);
     }
-    hipLaunchKernelGGL(kf, grid, dim3(kThreads), 0, st, ws, P, lk);
     mark(1);
   } else {
     const dim3 grid((unsigned)P.slices, (unsigned)P.rows);

@@ -90,7 +90,7 @@ def _batch(rows, V, dtype, sem, seed, masked):
     (64, 65536, _ffi.DTYPE_F32, _ffi.SEM_CBV2, True),      # four
     (43, 9000, _ffi.DTYPE_F32, _ffi.SEM_MLXLM, False),     # five: min-p alone
     (32, 65536, _ffi.DTYPE_BF16, _ffi.SEM_CBV2, False),    # eight: min-p alone
-    (150, 70001, _ffi.DTYPE_F32, _ffi.SEM_CBV2, False),    # past one round
+    (256, 70001, _ffi.DTYPE_F32, _ffi.SEM_CBV2, False),    # two launches
 ])
 def test_rows_from_lists(ctx, rows, V, dtype, sem, masked):
     cfg = _batch(rows, V, dtype, sem, rows + V, masked)
@@ -102,7 +102,7 @@ def test_rows_from_lists(ctx, rows, V, dtype, sem, masked):
     top_p = np.array([p["top_p"] < 1 for p in cfg["params"]])
     assert lists[~top_p].any() and lists[top_p].any() == (launch["slices"] <= 4)
     assert masked or not lists[6::10].any()  # (+inf logits, unless masked)
-    assert launch["fused"] == (5 if dtype == _ffi.DTYPE_F32 and rows == 150 else 1)
+    assert launch["fused"] == (5 if dtype == _ffi.DTYPE_F32 and rows == 256 else 1)
     ctx.read_status()
     _ffi.check(lib.lsamp_test_set_spin_limit(0, 16), "lsamp_test_set_spin_limit")
     try:

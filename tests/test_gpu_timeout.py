@@ -77,11 +77,11 @@ def test_slices_that_give_up_leave_their_work_to_the_last_arriver(ctx, rows):
 
 def test_fp32_batch_past_one_round_with_waits_given_up(ctx):
     """An fp32 batch with more slices than work-groups fit at once runs the
-    one-round kernel over the larger grid: rows exact with the hook on (every
-    slice that is not its row's last arriver leaves) and off."""
+    one-round kernel in two launches: rows exact with the hook on (every slice
+    that is not its row's last arriver leaves) and off."""
     import torch
     rng = np.random.default_rng(77)
-    rows, V = 150, 70001  # two slices a row, unaligned rows
+    rows, V = 256, 70001  # two slices a row, unaligned rows
     assert rows * 2 > torch.cuda.get_device_properties(0).multi_processor_count
     params = [W.resolve_cbv2(temperature=[0.8, 1.1, 0.0][r % 3], top_k=[0, 0, 30, 300][r % 4],
                              top_p=[0.9, 1.0][r % 2], vocab=V) for r in range(rows)]

@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 import oracle as O
+from common import rows_from_lists
 from lsamp import _ffi
 from lsamp import workloads as W
 
@@ -213,3 +214,50 @@ def test_residual_at_the_maximum_vocabulary(sigma, pkw):
     rej = [s for s in range(S) if o["accepted"][s] < Wn - 1]
     assert rej, "no rejection: the residual draw was not exercised"
     assert max(int(o["tokens"][s][o["accepted"][s]]) for s in rej) >= 262144
+
+
+@pytest.mark.parametrize("mode,dtype,S,Wn,V", [
+    (_ffi.VERIFY_RESIDUAL, _ffi.DTYPE_BF16, 9, 4, 4003),   # one round, four slices a row
+    (_ffi.VERIFY_TYPICAL, _ffi.DTYPE_F16, 16, 4, 30000),
+    (_ffi.VERIFY_EXACT, _ffi.DTYPE_F32, 16, 4, 30000),
+    (_ffi.VERIFY_RESIDUAL, _ffi.DTYPE_BF16, 12, 4, 40003),  # several rounds
+    (_ffi.VERIFY_RESIDUAL, _ffi.DTYPE_F32, 12, 4, 40003),   # fp32 past one round
+    (_ffi.VERIFY_RESIDUAL, _ffi.DTYPE_F32, 30, 4, 70001),
+    (_ffi.VERIFY_TYPICAL, _ffi.DTYPE_F32, 64, 3, 70001),
+])
+def test_windows_of_every_kind_of_row(ctx, mode, dtype, S, Wn, V):
+    """Sequences whose nuclei a few tokens hold, wide ones, top-k, min-p, greedy
+    and unfiltered ones side by side: rows that their slices' lists decide and
+    rows that exchange histograms, with what acceptance, the residual and the
+    bonus draw read of either."""
+    rng = np.random.default_rng(V + S)
+    t = rng.normal(0, 2, (S, Wn, V)).astype(np.float32)
+    t[np.arange(S) % 8 != 1] *= 1.5
+    pkw = [dict(temperature=0.7, top_p=0.9), dict(temperature=1.4, top_p=0.99),
+           dict(temperature=0.8, top_p=0.95), dict(temperature=0.9, min_p=0.05),
+           dict(temperature=0.6, top_p=0.8, min_p=0.01), dict(temperature=0.8, top_k=40),
+           dict(temperature=1.1), dict(temperature=0.0)]
+    for s in range(S):
+        if s % 8 in (0, 2, 4):  # a few tokens far ahead, in every slice
+            for j in range(Wn):
+                t[s, j, np.arange(24) * (V // 24) + rng.integers(0, V // 24, 24)] = \
+                    20 + 1.5 * rng.normal(size=24)
+    d = (t[:, : Wn - 1] + rng.normal(0, 1, (S, Wn - 1, V))).astype(np.float32)
+    if dtype == _ffi.DTYPE_BF16:
+        t, d = W.f32_to_bf16_bits(t), W.f32_to_bf16_bits(d)
+    elif dtype == _ffi.DTYPE_F16:
+        t, d = t.astype(np.float16).view(np.uint16), d.astype(np.float16).view(np.uint16)
+    params = W._params([W.resolve_cbv2(vocab=V, **pkw[s % 8]) for s in range(S)])
+    drafts = draw_drafts(d, dtype, params, rng.random((S, Wn - 1), dtype=np.float32))
+    u = rng.random((S, Wn), dtype=np.float32)
+    typical = mode == _ffi.VERIFY_TYPICAL
+    for rep in range(2):  # twice: the rows' words return to zero
+        g, o = run_both(ctx, mode, t, d if mode == _ffi.VERIFY_RESIDUAL else None, drafts, params, u,
+                        dtype, delta=0.2 if typical else 0.0)
+        check(g, o, f"mode {mode} rep {rep}", typical=typical)
+    assert 0 < g["accepted"].sum() < S * (Wn - 1)
+    lists = rows_from_lists(ctx, S * Wn).reshape(S, Wn)
+    if dtype == _ffi.DTYPE_F32 or S != 12:
+        assert lists[0::8].any() and lists[3::8].any()  # top-p rows, min-p rows
+    assert not lists[6::8].any()
+    assert ctx.read_status() == 0
