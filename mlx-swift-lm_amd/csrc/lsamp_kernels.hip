@@ -3281,9 +3281,8 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
             L.last = last ? 1 : 0;
           }
           __syncthreads();
-          if (L.last) {
-            if (L.wait == 0 && nucleus_row<DT>(ws, P, row, c, prm, nuc, L, rowp, sync, lpp))
-              return kJobLeave;
+          if (L.last && L.wait == 0) {
+            if (nucleus_row<DT>(ws, P, row, c, prm, nuc, L, rowp, sync, lpp)) return kJobLeave;
             // (its histogram from a re-read, as a claimed job: the registers
             // need not hold the slice through the row's work above)
             if (tid == 0) {
@@ -3292,7 +3291,11 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
             }
             return next_job(kBehalfStats, slice);
           }
+          // (a last arriver that finds the row wide already has the slice in
+          // its registers still: 64 rows x 151,936 bf16 whose slices differ,
+          // 62 us with a re-read, 53 without)
           if (L.wait != (int)kVerdictHistogram) return kJobLeave;
+          if (tid == 0 && L.last) L.x1 = 1;
           // (unless the last arriver has claimed this histogram)
           if (tid == 0) L.won = claim_bit(sync, kClaimStats + (uint32_t)slice) ? 1 : 0;
           __syncthreads();
