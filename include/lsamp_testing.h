@@ -21,11 +21,12 @@ extern "C" {
  * flight. */
 lsamp_status lsamp_test_set_spin_limit(int32_t device, int32_t polls);
 
-/* The launch plan of lsamp_top2 / lsamp_logprobs for `rows` rows of `vocab`
- * logits with `k` reported tokens on a device of `cus` compute units: slices a
- * row and tokens a slice.  No device work. */
+/* The launch plan of lsamp_top2 (`lse` 0) / lsamp_logprobs (1) for `rows` rows of
+ * `vocab` logits, 16-byte aligned or not, with `k` reported tokens on a device of
+ * `cus` compute units: slices a row and tokens a slice.  No device work. */
 lsamp_status lsamp_test_plan_rank(int32_t rows, int32_t vocab, int32_t dtype, int32_t k,
-                                  int32_t cus, int32_t* slices, int32_t* slice_len);
+                                  int32_t lse, int32_t aligned, int32_t cus, int32_t* slices,
+                                  int32_t* slice_len);
 
 /* For each of the first `rows` rows of the context's last sampling or
  * verification launch (not the top-k kernel's): 1 when the row was drawn from

@@ -213,24 +213,42 @@ RowMix row_mix(const lsamp_sample_args* a, int32_t slices) {
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// Slice option of a ranking launch: 16,384-token slices, or 32,768 where a row
-// would have more than 8 (fp32: 12; the merge of its lists is then twice as
-// wide: 32 x 151,936 bf16 top-2 11.0 us against 9.9), or where 16-bit rows make at least
-// three quarters of a work-group per CU of them anyway, most of a slice full
-// (192 x 128,256 log-probabilities 28.5 us against 21.4; fp32 rows, twice the
-// registers, gain nothing: 128 x 128,256 23.2 against 27.5).  Without a top k
-// there are no lists to merge: small slices while two work-groups a CU hold the
-// grid (6 x 151,936 chosen log-probability 6.2 us against 7.5).  A row never has
-// more than kRankMaxSlices of them: its records and arrivals are sized for that.
-void plan_rank(int32_t rows, int32_t vocab, int32_t dtype, int32_t k, int32_t cus,
-               int32_t* option, int32_t* slices) {
+// Slice option of a ranking launch.  Small slices spread a row over the chip
+// while few of them meet on a CU (three fit, of the largest two; fp32 32,768:
+// two), but each has a chain of its own and the merge of lists grows with their
+// number.  Rules from a sweep of 19 vocabularies x 17 row counts x 5 kinds of
+// call, fp32 and bf16 (figures: us with slices of 16,384 / 32,768 / 65,536):
+//  * small ones while one a CU holds the grid; while three do where lists cost
+//    less (fp32, no lists, or unaligned rows, bound by element loads: fp32 4 x
+//    200,065 top 5 14.1 / 18.1 / 26.1) and 32,768 would not bring the grid down
+//    to one a CU (64 x 128,256 bf16 top 5 14.2 / 12.5 / 15.3); past that fp32
+//    ones that pad a row less (224 x 100,352 28.0 / 29.9);
+//  * but at most 8 where lists of aligned rows are merged, 12 beside a log-sum-
+//    exp on half a work-group per CU (32 x 248,320 bf16 top two 13.5 / 10.5 / 10.8);
+//  * 65,536 for 16-bit grids past three 32,768 a CU where they pad a row no more
+//    or fit two a CU (114 x 262,144 top 5 35.5 / 25.4 / 22.8; 192 x 151,936 33.4 /
+//    26.8 / 29.9), or where lists of more than 8 slices would be merged.
+// A row never has more than kRankMaxSlices slices: its records and arrivals are
+// sized for that.
+void plan_rank(int32_t rows, int32_t vocab, int32_t dtype, int32_t k, bool lse, bool vec,
+               int32_t cus, int32_t* option, int32_t* slices) {
   const auto count = [vocab](int o) { return (vocab + rank_slice_len(o) - 1) / rank_slice_len(o); };
-  const bool lists = k > 0 || (int64_t)rows * count(0) > 2 * (int64_t)cus;
-  const bool wide = count(0) > kRankMaxSlices ||
-                    (lists && count(0) > (dtype == LSAMP_DTYPE_F32 ? 12 : 8)) ||
-                    (dtype != LSAMP_DTYPE_F32 && vocab > rank_slice_len(1) * 3 / 4 &&
-                     (int64_t)rows * count(1) >= (int64_t)cus * 3 / 4);
-  *option = wide ? 1 : 0;
+  const int32_t c0 = count(0), c1 = count(1), c2 = count(2);
+  const int64_t n0 = (int64_t)rows * c0, n1 = (int64_t)rows * c1, n2 = (int64_t)rows * c2;
+  const bool f32 = dtype == LSAMP_DTYPE_F32;
+  const int32_t most = !vec || k == 0 ? kRankMaxSlices : lse && n0 <= cus / 2 ? 12 : 8;
+  const bool fits = n0 <= cus ||
+                    (n0 <= 3 * (int64_t)cus
+                         ? (k == 0 && !vec) || (n1 > cus && (f32 || !vec || k == 0))
+                         : f32 && c0 < 2 * c1);
+  if (c0 <= most && fits)
+    *option = 0;
+  else if (f32 || !vec)
+    *option = 1;
+  else if (k > 0 && !lse && c1 > 8)
+    *option = 2;
+  else
+    *option = n1 > 3 * (int64_t)cus && (2 * c2 <= c1 || n2 <= 2 * (int64_t)cus) ? 2 : 1;
   *slices = count(*option);
 }
 
@@ -250,7 +268,7 @@ lsamp_status rank_common(lsamp_context* ctx, RankPlan& P, int32_t min_vocab, voi
   if (!P.logits) return fail(LSAMP_ERR_INVALID_ARGUMENT, "logits is NULL");
   const size_t es = P.dtype == LSAMP_DTYPE_F32 ? 4 : 2;
   P.vec = P.col_stride == 1 && aligned16(P.logits) && ((size_t)P.row_stride * es) % 16 == 0;
-  plan_rank(P.rows, P.vocab, P.dtype, P.k, ctx->cus, &P.option, &P.slices);
+  plan_rank(P.rows, P.vocab, P.dtype, P.k, P.lse != 0, P.vec != 0, ctx->cus, &P.option, &P.slices);
   P.part = ctx->rank_part;
   P.arrive = ctx->arrive_rank;
   DeviceGuard guard(ctx->device);
@@ -566,12 +584,13 @@ lsamp_status lsamp_test_set_spin_limit(int32_t device, int32_t polls) {
 }
 
 lsamp_status lsamp_test_plan_rank(int32_t rows, int32_t vocab, int32_t dtype, int32_t k,
-                                  int32_t cus, int32_t* slices, int32_t* slice_len) {
+                                  int32_t lse, int32_t aligned, int32_t cus, int32_t* slices,
+                                  int32_t* slice_len) {
   if (!slices || !slice_len) return fail(LSAMP_ERR_INVALID_ARGUMENT, "NULL argument");
   if (rows <= 0 || vocab <= 0 || vocab > kMaxVocab || cus <= 0)
     return fail(LSAMP_ERR_SHAPE, "rows %d / vocab %d / cus %d invalid", rows, vocab, cus);
   int32_t option = 0;
-  plan_rank(rows, vocab, dtype, k, cus, &option, slices);
+  plan_rank(rows, vocab, dtype, k, lse != 0, aligned != 0, cus, &option, slices);
   *slice_len = rank_slice_len(option);
   return ok();
 }

@@ -132,13 +132,13 @@ static_assert(kMaxRowChunks <= kThreads, "the draw keeps one chunk per thread");
 static_assert(kBins == 2 * kThreads, "the merge keeps two bins per thread");
 
 // Ranking of raw logits (exact top-k and log-probabilities).  One 512-thread
-// work-group per slice of a row; a slice is 16,384 or 32,768 tokens (option
-// 0 / 1, whatever the dtype: 32 / 64 tokens per thread).
+// work-group per slice of a row; a slice is 16,384 / 32,768 / 65,536 tokens
+// (option 0 / 1 / 2, whatever the dtype: 32 / 64 / 128 tokens per thread).
 constexpr int kRankMaxK = 32;
 constexpr int kRankMaxSlices = 16;
-constexpr int kRankOptions = 2;
+constexpr int kRankOptions = 3;
 constexpr int rank_slice_len(int option) { return 16384 << option; }
-static_assert(kRankMaxSlices * rank_slice_len(kRankOptions - 1) >= kMaxVocab,
+static_assert(kRankMaxSlices * rank_slice_len(1) >= kMaxVocab,
               "every vocabulary fits the larger slices");
 // Slice flags of the ranking.
 constexpr uint32_t kRankNaN = 1u;        // a NaN logit

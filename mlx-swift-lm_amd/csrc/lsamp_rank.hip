@@ -199,8 +199,15 @@ __device__ __forceinline__ int rank_in_sorted(const uint64_t (*a)[kRankMaxK], in
   return r;
 }
 
+// Slices of up to 256 bytes a thread keep their registers within 128, so that
+// two work-groups share a CU (but for the largest 16-bit ones of unaligned
+// rows, which would spill).
 template <int DT, int OPT, bool VEC>
-__global__ __launch_bounds__(kThreads) void k_rank(RankPlan P) {
+constexpr int rank_waves() {
+  return rank_slice_len(OPT) / kThreads * Vec<DT>::ESIZE <= 256 && VEC ? 4 : 2;
+}
+template <int DT, int OPT, bool VEC>
+__global__ __launch_bounds__(kThreads, (rank_waves<DT, OPT, VEC>())) void k_rank(RankPlan P) {
   using B = RankBits<DT>;
   using BT = Best<DT>;
   constexpr int N = B::N;
@@ -230,8 +237,16 @@ __global__ __launch_bounds__(kThreads) void k_rank(RankPlan P) {
 
   // ---- the slice's logits
   uint4 r[Q];
+  auto pack = [](const uint32_t* b) {
+    if constexpr (N == 4)
+      return make_uint4(b[0], b[1], b[2], b[3]);
+    else
+      return make_uint4(b[0] | (b[1] << 16), b[2] | (b[3] << 16), b[4] | (b[5] << 16),
+                        b[6] | (b[7] << 16));
+  };
+  const int32_t full = ns / N;  // whole vectors inside the slice
+  const int64_t cs = VEC ? 1 : P.col_stride;
   if constexpr (VEC) {
-    const int32_t full = ns / N;  // whole vectors inside the slice
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<char*>(rowp) + (size_t)s0 * ES, 0, full * 16, kBufferWord3);
 #pragma unroll
@@ -239,27 +254,7 @@ __global__ __launch_bounds__(kThreads) void k_rank(RankPlan P) {
       const auto w = __builtin_amdgcn_raw_buffer_load_b128(rs, tid * 16, q * kThreads * 16, 0);
       r[q] = make_uint4(w[0], w[1], w[2], w[3]);
     }
-    if (tail && (ns % N) != 0 && (full % kThreads) == tid) {
-      // the slice's last partial vector, element by element
-      const int qp = full / kThreads;
-      const int32_t i0 = s0 + full * N;
-      uint32_t b[N];
-#pragma unroll
-      for (int e = 0; e < N; ++e)
-        b[e] = full * N + e < ns ? load_raw_bits<DT>(rowp, i0 + e) : 0u;
-      uint4 v;
-      if constexpr (N == 4) {
-        v = make_uint4(b[0], b[1], b[2], b[3]);
-      } else {
-        v = make_uint4(b[0] | (b[1] << 16), b[2] | (b[3] << 16), b[4] | (b[5] << 16),
-                       b[6] | (b[7] << 16));
-      }
-#pragma unroll
-      for (int q = 0; q < Q; ++q)
-        if (q == qp) r[q] = v;
-    }
   } else {
-    const int64_t cs = P.col_stride;
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
       const int32_t l0 = (q * kThreads + tid) * N;
@@ -267,13 +262,20 @@ __global__ __launch_bounds__(kThreads) void k_rank(RankPlan P) {
 #pragma unroll
       for (int e = 0; e < N; ++e)
         b[e] = l0 + e < ns ? load_raw_bits<DT>(rowp, (int64_t)(s0 + l0 + e) * cs) : 0u;
-      if constexpr (N == 4) {
-        r[q] = make_uint4(b[0], b[1], b[2], b[3]);
-      } else {
-        r[q] = make_uint4(b[0] | (b[1] << 16), b[2] | (b[3] << 16), b[4] | (b[5] << 16),
-                          b[6] | (b[7] << 16));
-      }
+      r[q] = pack(b);
     }
+  }
+  if (tail && (ns % N) != 0 && (full % kThreads) == tid) {
+    // the slice's last partial vector, filled up with its first token
+    const int qp = full / kThreads;
+    uint32_t b[N];
+#pragma unroll
+    for (int e = 0; e < N; ++e)
+      b[e] = load_raw_bits<DT>(rowp, (int64_t)(s0 + full * N + (full * N + e < ns ? e : 0)) * cs);
+    const uint4 v = pack(b);
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+      if (q == qp) r[q] = v;
   }
   // while the logits stream in: the candidate list starts 0-padded
   if (k > 0) {
@@ -292,11 +294,14 @@ __global__ __launch_bounds__(kThreads) void k_rank(RankPlan P) {
   // operations a token, where a packed (key, position) per token took 10.
   uint32_t magmax = 0;
   {
-    constexpr uint32_t M2 = B::W == 32 ? B::MAG : B::MAG * 0x10001u;
+    constexpr uint32_t M2 = B::MAG * 0x10001u;  // (16-bit types)
     if constexpr (B::W == 32) {
+      // (shifted: with a mask the compiler keeps all of its results for the
+      // passes below, 25 registers past the two work-groups' share)
 #pragma unroll
       for (int q = 0; q < Q; ++q)
-        magmax = max(max(max(magmax, r[q].x & M2), r[q].y & M2), max(r[q].z & M2, r[q].w & M2));
+        magmax = max(max(max(magmax, r[q].x << 1), r[q].y << 1), max(r[q].z << 1, r[q].w << 1));
+      magmax >>= 1;
     } else {
       typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
       u16x2 m2 = {0, 0};
@@ -310,26 +315,20 @@ __global__ __launch_bounds__(kThreads) void k_rank(RankPlan P) {
       magmax = max((uint32_t)m2.x, (uint32_t)m2.y);
     }
   }
-  // places past the slice's tokens read -inf from here on (they come after
-  // the thread's own tokens, so the first maximum is a token's)
-  if (tail) {
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-      const int32_t rem = ns - (q * kThreads + tid) * N;
-      exclude_elems<DT>(r[q], ~0u << (uint32_t)(rem < 0 ? 0 : (rem > N ? N : rem)) &
-                                  ((1u << N) - 1u));
-    }
-  }
+  // (places past the slice's tokens: a partial vector's repeat its first token,
+  // after that one in order; whole vectors read zero, which raises no magnitude,
+  // and are passed over here)
   typename BT::T best = 0;
   const bool safe = magmax > B::INF;  // a NaN: again, element by element
-  if (!safe && tid * N < ns) {
+  const int32_t lim = ns - tid * N;  // the slice's tokens from the thread's first on
+  if (!safe && lim > 0) {
     uint4 bv = r[0];
     int bq = 0;
     float bm = vec_max_nn<DT>(r[0]);
 #pragma unroll
     for (int q = 1; q < Q; ++q) {
       const float m = vec_max_nn<DT>(r[q]);
-      const bool up = m > bm;
+      const bool up = m > bm && q * kThreads * N < lim;
       bm = up ? m : bm;
       bq = up ? q : bq;
       bv.x = up ? r[q].x : bv.x;
@@ -377,13 +376,24 @@ __global__ __launch_bounds__(kThreads) void k_rank(RankPlan P) {
   // log-sum-exp partial: sum exp(x - m_t) over the thread's finite logits
   float s_t = 0.f;
   if (P.lse && m_t > kNegInf && m_t < kPosInf) {
-    if (!safe) {
+    auto term = [m_t](float x) { return __builtin_amdgcn_exp2f((x - m_t) * kLog2e); };
+    if (!safe && !tail) {
 #pragma unroll
       for (int q = 0; q < Q; ++q) {
 #pragma unroll
+        for (int e = 0; e < N; ++e) s_t += term(bits_value<DT>(elem_bits<DT>(r[q], e)));
+      }
+    } else if (!safe) {
+      // (the last slice; its vectors opaque, so that the compiler does not keep
+      // the three loops' shared conversions for all of them)
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        uint4 w = r[q];
+        asm volatile("" : "+v"(w.x), "+v"(w.y), "+v"(w.z), "+v"(w.w));
+#pragma unroll
         for (int e = 0; e < N; ++e) {
-          const float x = bits_value<DT>(elem_bits<DT>(r[q], e));
-          s_t += __builtin_amdgcn_exp2f((x - m_t) * kLog2e);
+          const float v = term(bits_value<DT>(elem_bits<DT>(w, e)));
+          s_t += q * kThreads * N + e < lim ? v : 0.f;
         }
       }
     } else {
@@ -393,8 +403,7 @@ __global__ __launch_bounds__(kThreads) void k_rank(RankPlan P) {
         for (int e = 0; e < N; ++e) {
           const uint32_t b = elem_bits<DT>(r[q], e);
           const bool ok = (q * kThreads + tid) * N + e < ns && (b & B::MAG) <= B::INF;
-          const float x = ok ? bits_value<DT>(b) : kNegInf;
-          s_t += __builtin_amdgcn_exp2f((x - m_t) * kLog2e);
+          s_t += term(ok ? bits_value<DT>(b) : kNegInf);
         }
       }
     }
@@ -586,7 +595,10 @@ template <int DT>
 void launch_rank_dt(const RankPlan& P, hipStream_t st) {
   switch (P.option) {
     case 0: launch_rank_t<DT, 0>(P, st); break;
-    default: launch_rank_t<DT, 1>(P, st); break;
+    case 1: launch_rank_t<DT, 1>(P, st); break;
+    default:  // (16-bit types; an fp32 one, at a work-group a CU, is never the best)
+      if constexpr (DT != LSAMP_DTYPE_F32) launch_rank_t<DT, 2>(P, st);
+      break;
   }
 }
 

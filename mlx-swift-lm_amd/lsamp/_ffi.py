@@ -321,7 +321,7 @@ def load_library(path: str | None = None):
     lib.lsamp_test_set_spin_limit.restype = c_int32
     lib.lsamp_test_rows_from_lists.argtypes = [c_void_p, c_int32, POINTER(c_int32)]
     lib.lsamp_test_rows_from_lists.restype = c_int32
-    lib.lsamp_test_plan_rank.argtypes = [c_int32] * 5 + [POINTER(c_int32)] * 2
+    lib.lsamp_test_plan_rank.argtypes = [c_int32] * 7 + [POINTER(c_int32)] * 2
     lib.lsamp_test_plan_rank.restype = c_int32
     lib.lsamp_context_last_launch.argtypes = [c_void_p, POINTER(LaunchInfo)]
     lib.lsamp_context_last_launch.restype = c_int32

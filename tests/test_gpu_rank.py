@@ -178,3 +178,57 @@ def test_chosen_log_probability_of_the_largest_vocabularies(vocab, dtype):
     finally:
         torch.cuda.synchronize()
         c.close()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("vocab", [4099, 16389, 147461, 212995])  # small slices, and large ones
+def test_largest_values_of_a_thread(ctx, vocab, dtype):
+    """The thread's best token is the first of its largest value: ties across its
+    vectors and inside one, zeros of both signs, denormals, in full slices and
+    in a last slice that begins or ends inside a vector."""
+    rng = np.random.default_rng(vocab + dtype)
+    rows, n = 8, 4 if dtype == F32 else 8
+    tiny = {F32: 1e-42, F16: 6e-8, BF16: 1e-39}[dtype]
+    x = np.minimum(rng.normal(-3.0, 1.0, (rows, vocab)), -0.5).astype(np.float32)
+    step = 512 * n  # the same thread's next vector
+    last = (vocab - 1) // 16384 * 16384
+    x[0, [n * 5, n * 5 + 1, (n * 5 + step) % vocab]] = 4.0
+    x[1, [3, 3 + n - 1, (3 + step) % vocab, vocab - 1]] = 0.0
+    x[1, 3] = -0.0
+    x[2, rng.choice(vocab, 30, replace=False)] = rng.integers(1, 5, 30) * tiny
+    x[3, rng.choice(vocab, 30, replace=False)] = -rng.integers(1, 5, 30) * tiny
+    x[4, last:] = -rng.integers(0, 3, vocab - last) * tiny
+    x[5, vocab - 3:] = [-0.0, 0.0, -0.0]
+    x[6] = -0.0
+    x[6, rng.choice(vocab, 20, replace=False)] = 0.0
+    x[7, last:] = 1.0
+    b = to_bits(x, dtype)
+    for off in (0, 1):
+        check_top2(ctx, b, dtype, rows - 1, vocab, vocab, 1, offset=off, label=f"offset {off}")
+        check_logprobs(ctx, b, dtype, rows - 1, vocab, vocab, 1, 20, offset=off,
+                       tokens=rng.integers(0, vocab, rows - 1).astype(np.int32), label=f"offset {off}")
+    check_top2(ctx, b, dtype, rows, vocab, vocab, 1, label="all rows")
+
+
+@pytest.mark.parametrize("dtype", [BF16, F16])
+def test_slices_of_the_largest_size(dtype):
+    """Batches that take 65,536-token slices: aligned rows whose last slice ends
+    inside a vector, with special values in some."""
+    import ctypes
+    from lsamp import _ffi
+    from lsamp.api import Context
+    rng = np.random.default_rng(dtype)
+    rows, vocab, stride = 100, 262132, 262136
+    g, n = ctypes.c_int32(), ctypes.c_int32()
+    c = Context(0, max_rows=rows, max_vocab=vocab)
+    try:
+        _ffi.check(c.lib.lsamp_test_plan_rank(rows, vocab, dtype, 5, 1, 1, 256,
+                                              ctypes.byref(g), ctypes.byref(n)), "plan")
+        assert n.value == 65536
+        b = batch(rng, rows, stride, dtype)
+        tok = rng.integers(0, vocab, rows).astype(np.int32)
+        for _ in range(2):
+            check_logprobs(c, b, dtype, rows, vocab, stride, 1, 5, tokens=tok, label="top 5")
+        check_top2(c, b, dtype, rows, vocab, stride, 1, label="top two")
+    finally:
+        c.close()
