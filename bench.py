@@ -100,8 +100,8 @@ def parse():
 
 def sample_kernel_name(launch):
     """The kernel(s) one sampling step launched (lsamp_launch_info.fused:
-    2 the one-pass top-k kernel, 1 the fused kernel, 5 the same in several
-    launches, 0 the two-kernel split)."""
+    2 the one-pass top-k kernel, 1 the fused kernel, 5 the same on a
+    larger grid, 0 the two-kernel split)."""
     return {5: "k_fused", 4: "k_fused", 3: "k_topk", 2: "k_topk", 1: "k_fused"}.get(launch["fused"],
                                                                        "k_stats+k_select")
 

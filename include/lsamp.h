@@ -331,8 +331,8 @@ lsamp_status lsamp_context_read_timing(lsamp_context* ctx, double* stats_ms, dou
  * (each slice of a row publishes its best keys; the slice that starts last
  * merges and draws; no co-residency needed), else one kernel (the slices of
  * a row hand their results to each other while the logits stay in registers;
- * its grid fits on the device at once; an fp32 batch larger than that takes
- * several launches, or the split kernels).  FUSED never takes the top-k
+ * its grid fits on the device at once, but for fp32 batches larger than that,
+ * which may also take the split kernels).  FUSED never takes the top-k
  * kernel; SPLIT runs two kernels with no co-residency requirement (the
  * second re-reads each slice from L2).  All give identical results. */
 #define LSAMP_MODE_AUTO 0
@@ -356,9 +356,9 @@ lsamp_status lsamp_context_read_status(lsamp_context* ctx, uint32_t* bits);
 
 /* Launch shape of the context's last lsamp_sample call (diagnostics; no
  * device work): fused with raw log-probabilities (4, lsamp_step), top-k with
- * raw log-probabilities (3, lsamp_step), top-k (2), fused in one launch (1),
- * fused in several launches (5: fp32 batches past one round), split kernels
- * (0); slices per row, tokens per slice, rows per round of the fused
+ * raw log-probabilities (3, lsamp_step), top-k (2), fused on a grid that
+ * fits the device at once (1), fused on a larger one (5: fp32 batches), split
+ * kernels (0); slices per row, tokens per slice, rows per round of the fused
  * grid, work-groups per kernel launch. */
 typedef struct lsamp_launch_info {
   int32_t fused;

@@ -154,26 +154,24 @@ void plan_slices(int32_t rows, int32_t vocab, int32_t slots, int32_t* slices, in
   *nchunks = nch;
 }
 
-// An fp32 batch past one round of `slots` work-groups (the several-rounds form
-// is not built for the fp32 slab: it would not fit the registers): as few
-// launches of the one-round kernel as the longest slices allow, the rows spread
-// evenly over them, each on a grid that fits the device at once.  Returns the
-// rows of a launch, or 0, the plan as it was, where several launches would leave
-// more than a sixteenth of their slots idle: the split kernels' grid has no such
-// gaps (verification, 224 rows x 151,936 in three launches of 75, 433 us, split
-// 396; 128 x 100,000 in one launch 40, split 44).  (One launch over a larger grid
-// starts a row's slices apart, and the last one did the others' selects:
-// 128 rows x 151,936 verified without filters 397 us, the split kernels 252.)
-int32_t plan_launches(int32_t rows, int32_t vocab, int32_t slots, int32_t* slices,
-                      int32_t* slice_len, int32_t* nchunks) {
+// Slices of an fp32 batch past one round of `slots` work-groups, which runs the
+// one-round kernel over a larger grid (the several-rounds form is not built for
+// the fp32 slab: it would not fit the registers): the rows spread evenly over as
+// few rounds as the longest slices allow, with as many slices as fill a round
+// (128 rows x 151,936: two rounds of 64 rows x 4 slices).  Returns the rows of a
+// round, or 0, the plan as it was, where more than a sixteenth of several rounds
+// would stay idle: the split kernels are steadier there (171 x 151,936 of wide
+// nuclei 307 us, split 246; 128 x 100,000 in one round 40, split 44).
+int32_t plan_rounds(int32_t rows, int32_t vocab, int32_t slots, int32_t* slices,
+                    int32_t* slice_len, int32_t* nchunks) {
   const int32_t g_min = (vocab + kMaxSliceLen - 1) / kMaxSliceLen;
-  const int32_t most = slots / g_min;  // rows a launch holds
-  const int32_t launches = (rows + most - 1) / most;
-  const int32_t per = (rows + launches - 1) / launches;
+  const int32_t most = slots / g_min;  // rows a round holds
+  const int32_t rounds = (rows + most - 1) / most;
+  const int32_t per = (rows + rounds - 1) / rounds;
   int32_t g = 0, len = 0, nch = 0;
   // (as many slots as whole slices of those rows fill)
   plan_slices(per, vocab, slots / per * per, &g, &len, &nch);
-  if (launches > 1 && 16 * (int64_t)rows * g < 15 * (int64_t)launches * slots) return 0;
+  if (rounds > 1 && 16 * (int64_t)rows * g < 15 * (int64_t)rounds * slots) return 0;
   *slices = g;
   *slice_len = len;
   *nchunks = nch;
@@ -358,9 +356,9 @@ lsamp_status lsamp::sample_step(const WorkspaceViews& v, const DeviceShape& d, i
   // (the top-k kernel: one work-group per CU is enough, and fewer slices per
   // row mean a shorter merge)
   plan_slices(a->rows, a->vocab, topk ? d.cus : slots, &P.slices, &P.slice_len, &P.nchunks);
-  // An fp32 batch past one round of the grid: launches of one round each, where
-  // at least half of its rows are drawn from lists (128 rows x 151,936 with
-  // top-p: 75 us, the split kernels, which read every slice twice, 101).  Others
+  // An fp32 batch past one round of the grid: one kernel over a larger grid,
+  // where at least half of its rows are drawn from lists (128 rows x 151,936 with
+  // top-p: 69 us, the split kernels, which read every slice twice, 101).  Others
   // keep the split kernels, and so does a batch that asks for raw
   // log-probabilities.
   bool one = !topk && bpc > 0 && slots >= P.slices;
@@ -370,7 +368,7 @@ lsamp_status lsamp::sample_step(const WorkspaceViews& v, const DeviceShape& d, i
   if (over) {
     int32_t slices = P.slices, slice_len = P.slice_len;
     per = lp && lp->k >= 0 ? 0
-                           : plan_launches(a->rows, a->vocab, slots, &slices, &slice_len, &P.nchunks);
+                           : plan_rounds(a->rows, a->vocab, slots, &slices, &slice_len, &P.nchunks);
     const RowMix there = per > 0 ? row_mix(a, slices) : RowMix{false, false};
     one = there.lists;
     if (one) {  // (also in split mode: the same slices)
@@ -451,8 +449,9 @@ lsamp_status lsamp::sample_step(const WorkspaceViews& v, const DeviceShape& d, i
   last->slice_len = P.slice_len;
   last->rows_per_round = P.rows_per_round;
   last->grid = topk ? (P.rows + 7) / 8 * 8 * P.slices
-                    : (P.fused & kPlanFused) ? (P.rows < P.rows_per_round ? P.rows : P.rows_per_round) * P.slices
-                              : P.rows * P.slices;
+                    : (P.fused & kPlanFused) && !over
+                        ? (P.rows < P.rows_per_round ? P.rows : P.rows_per_round) * P.slices
+                        : P.rows * P.slices;
   const int err =
       topk ? launch_topk(P, v.topk, lpk, stream, ev)
            : launch_sample(v.ws, P, lp_sample ? &flp : nullptr, stream, ev);
@@ -1133,7 +1132,7 @@ lsamp_status lsamp_verify(lsamp_context* ctx, const lsamp_verify_args* a, void* 
   int32_t per = slots / P.slices;
   // (fp32 past one round; nothing is known of the rows here)
   if (one && a->dtype == LSAMP_DTYPE_F32 && (int64_t)P.rows * P.slices > slots) {
-    per = plan_launches(P.rows, P.vocab, slots, &P.slices, &P.slice_len, &P.nchunks);
+    per = plan_rounds(P.rows, P.vocab, slots, &P.slices, &P.slice_len, &P.nchunks);
     one = per > 0;
   }
   P.fused = one && ctx->mode != LSAMP_MODE_SPLIT;

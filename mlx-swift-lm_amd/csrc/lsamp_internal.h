@@ -325,8 +325,7 @@ struct SamplePlan {
   int32_t nchunks;
   int32_t aligned;         // 16-byte vector loads allowed
   int32_t fused;           // kPlanFused, kPlanLists
-  int32_t rows_per_round;  // fused: rows processed per round of the grid (fp32: per launch)
-  int32_t row0;            // fused, one round: the launch's first row
+  int32_t rows_per_round;  // fused: rows processed per round of the grid (fp32: that fit at once)
   const void* logits;
   const void* logits2;     // rows >= rows_split read logits2 (MTP draft rows)
   int32_t rows_split;

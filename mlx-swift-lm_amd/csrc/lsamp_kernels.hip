@@ -128,13 +128,21 @@ __device__ __forceinline__ int wait_exchange(const Workspace& ws, const uint32_t
   }
 }
 
-// A slice without filters is at the exchange after one pass, before the row's
-// next slices have started where work-groups take several tasks (they end in
-// bursts, up to a finalize apart).  It waits this long (thread 0, about 25 us)
-// for their start rather than leave its select to the last one: 200 rows x
-// 151,936 bf16 360 us without this wait, 255 with it, 305 when such rows built
-// histograms as all others do.  True when every slice has started.
-constexpr int kStartPolls = 128;
+// Where a grid is larger than the device (fp32), or work-groups take several
+// tasks, a row's slices may start apart: work-groups end in bursts, a select and
+// a finalize apart.  A slice that reaches an exchange before its row's next
+// slices have started then waits this long (thread 0, about 100 us) for their
+// start rather than leave its work to the last one: in the former case every
+// slice (fp32 128 rows x 151,936 of wide nuclei 316 us without this wait, 210
+// with it), in the latter those of rows without filters, which are there after
+// one pass (200 rows x 151,936 bf16 360 us, 255 with it, 305 when such rows
+// built histograms as all others do).  128 polls did for the latter, not for the
+// former (320).  True when every slice has started.
+constexpr int kStartPolls = 512;
+template <int DT>
+__device__ __forceinline__ bool starts_apart(const SamplePlan& P) {
+  return DT == LSAMP_DTYPE_F32 && P.rows > P.rows_per_round;
+}
 __device__ __forceinline__ bool wait_started(const uint32_t* sync, int G) {
   if (__hip_atomic_load(&g_spin_test, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) > 0) return false;
   for (int it = 0; it < kStartPolls; ++it) {
@@ -3275,7 +3283,8 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
           if (tid == 0) {
             const bool last = (word & kArriveMask) + 1u == (uint32_t)G;
             int w = (word & kWideMask) != 0u ? (int)kVerdictHistogram : 0;
-            if (w == 0 && !last && (word >> 16) >= (uint32_t)G)
+            if (w == 0 && !last &&
+                ((word >> 16) >= (uint32_t)G || (starts_apart<DT>(P) && wait_started(sync, G))))
               w = wait_verdict(ws, sync, kClaimStats + (uint32_t)slice);
             L.wait = w;
             L.last = last ? 1 : 0;
@@ -3633,7 +3642,8 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
         int w = 1;
         if (!last && !L.x1) {
           const bool all =
-              started >= (uint32_t)G || (open_row(P, c, prm) && wait_started(sync, G));
+              started >= (uint32_t)G ||
+              ((starts_apart<DT>(P) || open_row(P, c, prm)) && wait_started(sync, G));
           w = all ? wait_exchange(ws, sync, kArriveHists, (uint32_t)G, (uint32_t)own) : 0;
           if (w == 1)
             claimed = __hip_atomic_fetch_or(sync + kSyncClaims, 1u << own, __ATOMIC_RELAXED,
@@ -3966,8 +3976,8 @@ __device__ __forceinline__ uint32_t run_task(const Workspace& ws, const SamplePl
 
 // ================================================================ kernels
 // ONE: a work-group per task (no loop over rounds, so nothing is hoisted out
-// of one and spilled before the first load): every row of the launch, from
-// row0 on, fits one round of the grid.
+// of one and spilled before the first load): every row fits one round of the
+// grid, or (fp32) the grid is larger than the device.
 // NUC (with ONE): nucleus rows go through lists.  A batch whose host copy of the
 // parameters shows no such row runs the kernel without that code, which costs
 // the other rows 0.5 to 1.5 us by its registers and its size.
@@ -3982,10 +3992,8 @@ __global__ __launch_bounds__(kThreads) void k_fused(Workspace wsk, SamplePlan Pk
   const Workspace ws = in_sgprs(wsk);
   const SamplePlan P = in_sgprs(Pk);
   const int G = P.slices;
-  const int rowslot = (int)blockIdx.x / G;
-  const int slice = (int)blockIdx.x % G;
   if (ONE) {
-    const int row = P.row0 + rowslot;
+    const int row = (int)blockIdx.x / G, slice = (int)blockIdx.x % G;
     if (row < P.rows) {
       const uint32_t out = run_task<DT, kFused, LP, NUC>(ws, P, row, slice, L, Lk);
       if (threadIdx.x == 0) clear_if_last(ws, row, G, out);
@@ -4094,21 +4102,17 @@ int launch_dt(const Workspace& ws, const SamplePlan& P, const FusedLp* lp, hipSt
     const bool nuc = (P.fused & kPlanLists) != 0;
     auto kf = lp ? (nuc ? k_fused<DT, true, true, true> : k_fused<DT, true, true, false>)
                  : (nuc ? k_fused<DT, true, false, true> : k_fused<DT, true, false, false>);
-    auto launch = [&](const SamplePlan& Pl, int rows) {
-      hipLaunchKernelGGL(kf, dim3((unsigned)(rows * P.slices)), dim3(kThreads), 0, st, ws, Pl, lk);
-    };
-    const int per = P.rows < P.rows_per_round ? P.rows : P.rows_per_round;
     // (fp32 steps have no several-rounds instantiation: with the fp32 slab it
-    // does not fit the registers)
-    if constexpr (DT == LSAMP_DTYPE_F32) {
-      SamplePlan Pl = P;
-      for (Pl.row0 = 0; Pl.row0 < P.rows; Pl.row0 += per)
-        launch(Pl, P.rows - Pl.row0 < per ? P.rows - Pl.row0 : per);
-    } else {
-      if (P.rows > P.rows_per_round)
+    // does not fit the registers.  A batch past one round gets a work-group per
+    // task, which the dispatcher starts in order as others end)
+    int rows = P.rows;
+    if constexpr (DT != LSAMP_DTYPE_F32) {
+      if (P.rows > P.rows_per_round) {
         kf = lp ? k_fused<DT, false, true, false> : k_fused<DT, false, false, false>;
-      launch(P, per);
+        rows = P.rows_per_round;
+      }
     }
+    hipLaunchKernelGGL(kf, dim3((unsigned)(rows * P.slices)), dim3(kThreads), 0, st, ws, P, lk);
     mark(1);
   } else {
     const dim3 grid((unsigned)P.slices, (unsigned)P.rows);

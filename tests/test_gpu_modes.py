@@ -104,8 +104,8 @@ def test_fp32_steps_of_several_rounds_run_split(ctx):
 
 def test_fp32_list_rows_past_one_round_run_fused(ctx):
     """Such a batch of argmax and top-k rows, which lists decide, takes the
-    fused kernel in several launches (kind 5) of the same rows, each on a grid
-    that fits the device, with the split kernels' results."""
+    fused kernel on a grid larger than the device (kind 5), rows spread evenly
+    over its rounds, with the split kernels' results."""
     cfg = _many_rounds_cfg(_ffi.DTYPE_F32)
     cfg["params"] = W._params([W.resolve_cbv2(temperature=[0.0, 0.7, 1.0][r % 3], top_k=[40, 5, 90][r % 3],
                                               top_p=[1.0, 0.9][r % 2], vocab=cfg["vocab"])
@@ -119,7 +119,8 @@ def test_fp32_list_rows_past_one_round_run_fused(ctx):
     finally:
         ctx.set_mode(_ffi.MODE_AUTO)
     per = launch["rows_per_round"]
-    assert launch["fused"] == 5 and launch["grid"] == per * launch["slices"] <= 256, launch
+    assert launch["fused"] == 5 and launch["grid"] == cfg["rows"] * launch["slices"], launch
+    assert per * launch["slices"] <= 256, launch
     assert per < cfg["rows"] <= -(-cfg["rows"] // per) * per, launch
 
 

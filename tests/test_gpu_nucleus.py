@@ -90,7 +90,7 @@ def _batch(rows, V, dtype, sem, seed, masked):
     (64, 65536, _ffi.DTYPE_F32, _ffi.SEM_CBV2, True),      # four
     (43, 9000, _ffi.DTYPE_F32, _ffi.SEM_MLXLM, False),     # five: min-p alone
     (32, 65536, _ffi.DTYPE_BF16, _ffi.SEM_CBV2, False),    # eight: min-p alone
-    (256, 70001, _ffi.DTYPE_F32, _ffi.SEM_CBV2, False),    # two launches
+    (256, 70001, _ffi.DTYPE_F32, _ffi.SEM_CBV2, False),    # past one round
 ])
 def test_rows_from_lists(ctx, rows, V, dtype, sem, masked):
     cfg = _batch(rows, V, dtype, sem, rows + V, masked)

@@ -77,8 +77,8 @@ def test_slices_that_give_up_leave_their_work_to_the_last_arriver(ctx, rows):
 
 def test_fp32_batch_past_one_round_with_waits_given_up(ctx):
     """An fp32 batch with more slices than work-groups fit at once runs the
-    one-round kernel in two launches: rows exact with the hook on (every slice
-    that is not its row's last arriver leaves) and off."""
+    one-round kernel over the larger grid: rows exact with the hook on (every
+    slice that is not its row's last arriver leaves) and off."""
     import torch
     rng = np.random.default_rng(77)
     rows, V = 256, 70001  # two slices a row, unaligned rows
