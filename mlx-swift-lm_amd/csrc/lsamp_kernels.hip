@@ -2333,9 +2333,11 @@ __device__ __forceinline__ void wave_reach(float v, float top, int m0, int m1, f
   r1 = nf >= m1 ? lo1 : kNegInf;
 }
 // The share of a wave's 64 thread maxima that its list is sized by: few (which
-// stay within the last arriver's first round trip), or what the list holds.
+// stay within the last arriver's first round trip), or what the list holds (60
+// of 64: 170 tokens, in 256 waves of Gaussian rows at most 240 of the 256 that
+// fit; at 61 some wave of a batch overflowed, and its row paid for both paths).
 __device__ __forceinline__ int nucleus_share(int seg, bool few) {
-  return few ? (seg >= 8 ? 40 : 25) : (seg >= 9 ? 63 : seg == 8 ? 61 : 51);
+  return few ? (seg >= 8 ? 40 : 25) : (seg >= 9 ? 63 : seg == 8 ? 60 : 51);
 }
 
 // This wave's part of a slice's list: the tokens at or above `tau` (and
@@ -3201,8 +3203,10 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
           if ((tid & 63) == 0) L.redu[wv] = ze;
         }
         // The list's size (entries apart): few when the mass below their
-        // threshold is well below what top-p drops, else many, unless even
-        // theirs leaves out more than top-p drops.  The thresholds are the
+        // threshold is at most half of what top-p drops (the estimate is off by
+        // up to a quarter, and slices differ: at 0.7 some row of a batch was
+        // listed in vain, 68 us a batch instead of 31), else many, unless even
+        // theirs leaves out nearly what top-p drops.  The thresholds are the
         // waves' averaged (a wave with too few maxima lists all it has down to
         // `low`), waves far below the slice's maximum apart.
         const float low = (nuc & kNucP) != 0 ? xmax - kNucRange / lgz : kNegInf;
@@ -3220,8 +3224,8 @@ __device__ __forceinline__ int slice_job(const Workspace& ws, const SamplePlan& 
           const float u_few = sum8(nw.z_few * f) * (float)kThreads;
           const float u_many = sum8(nw.z_many * f) * (float)kThreads;
           const float s_few = sum8(nw.n_few), s_many = sum8(nw.n_many);
-          const bool is_few = u_few <= 0.7f * drop * s_few;
-          wide = !is_few && u_many > 0.85f * drop * s_many;
+          const bool is_few = u_few <= 0.5f * drop * s_few;
+          wide = !is_few && u_many > 0.8f * drop * s_many;
           const float qw = is_few ? nw.q_few : nw.q_many;
           const bool near = qw > kNegInf && nw.hi > low;
           const float sum = sum8(near ? qw : 0.0f);

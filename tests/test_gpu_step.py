@@ -16,6 +16,7 @@ import numpy as np
 import pytest
 
 import oracle as O
+from common import rows_from_lists
 from lsamp import _ffi
 from lsamp import workloads as W
 from lsamp.history import Cbv2RowState, csr
@@ -205,7 +206,8 @@ def _fused_params(rows, vocab):
 
 @pytest.mark.parametrize("dtype", [F32, BF16], ids=["f32", "bf16"])
 @pytest.mark.parametrize("vocab,k,rows", [(151936, 0, 12), (151936, 20, 12), (151936, 32, 12),
-                                          (40003, 1, 12), (40003, 20, 12), (151936, 20, 80)])
+                                          (40003, 1, 12), (40003, 20, 12), (151936, 20, 80),
+                                          (40003, 0, 64), (40003, 20, 64)])
 def test_step_logprobs_in_the_fused_pass(dtype, vocab, k, rows):
     """The fused sampling kernel's raw log-probabilities (launch kind 4: no
     second pass over the logits) against the oracle's raw ranking
@@ -214,7 +216,8 @@ def test_step_logprobs_in_the_fused_pass(dtype, vocab, k, rows):
     +inf, all -inf, tied, signed-zero rows; rows that are not 16-byte aligned
     (odd vocabularies); 80 rows take the fused grid in several rounds (16-bit
     logits; fp32 steps that do not fit one round run split, with the second
-    pass)."""
+    pass); 64 rows make slices whose lists draw the top-p rows, the ranking
+    beside that draw."""
     import torch
     from lsamp.api import Context, PenaltyTable
     ctx = Context(0, max_rows=rows, max_vocab=vocab)
@@ -246,6 +249,8 @@ def test_step_logprobs_in_the_fused_pass(dtype, vocab, k, rows):
         else:
             assert launch["fused"] == 4, launch
             assert rows != 80 or launch["rows_per_round"] < rows, launch
+        if rows == 64:
+            assert rows_from_lists(ctx, rows)[8::4].any()
         tok = out["tokens"].cpu().numpy()
         ref = O.rank(np.ascontiguousarray(bits).reshape(-1), dtype=dtype, k=k, raw_values=False,
                      rows=rows, vocab=vocab, row_stride=vocab, col_stride=1, tokens=tok)
