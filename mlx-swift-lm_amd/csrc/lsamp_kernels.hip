@@ -2438,14 +2438,17 @@ __device__ __forceinline__ void nucleus_list(const Workspace& ws, const SamplePl
     }
     fits = n <= cap;
   }
-  float listed = 0.0f;
+  // (2^40 fixed point: the same in any order, which the entry table's depends on
+  // atomics for)
+  uint64_t listed = 0ull;
   const float lg = (float)(1.4426950408889634 / c.tf);
   if (fits) {
     __builtin_amdgcn_wave_barrier();
     for (int i = lane; i < n; i += 64) {
       const uint64_t k = lst[i];
       st_coherent(nucleus_key(ws, row, lay.shift, slice, (wv << lay.seg) + i), k);
-      listed += __builtin_amdgcn_exp2f((__uint_as_float((uint32_t)(k >> 32)) - xmax) * lg);
+      listed += (uint64_t)(__builtin_amdgcn_exp2f((__uint_as_float((uint32_t)(k >> 32)) - xmax) * lg) *
+                           0x1p40f);
     }
   }
   listed = wave_sum(listed);
@@ -2456,7 +2459,7 @@ __device__ __forceinline__ void nucleus_list(const Workspace& ws, const SamplePl
     st_coherent(&head[kWaves + wv], ze);
     L.hn[wv] = fits ? n : -1;
     L.hx[wv] = below;
-    L.hz[wv] = listed;
+    L.hz[wv] = (double)listed * 0x1p-40;
   }
 }
 
