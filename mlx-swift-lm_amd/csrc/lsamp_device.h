@@ -298,8 +298,8 @@ __device__ __forceinline__ float key_to_float(uint32_t k) {
   return __uint_as_float(b);
 }
 
-// Histogram bin of a transformed logit: floor(x * c32) with c32 = 32 / T,
-// clamped so the integer conversion is defined for any finite x.
+// Histogram bin of a transformed logit: floor(x * c32) with c32 = 32 (bins of
+// 1/32), clamped so the integer conversion is defined for any finite x.
 __device__ __forceinline__ float bin_pos(float x, float c32) {
   return __builtin_amdgcn_fmed3f(x * c32, -1.0e9f, 1.0e9f);
 }

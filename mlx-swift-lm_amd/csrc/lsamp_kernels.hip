@@ -295,7 +295,7 @@ struct ShortLds {
 };
 // A nucleus row's slice, one wave's maxima and masses (see slice_job).
 struct NucWave {
-  float hi, q_few, q_many, z_few, z_many, n_few, n_many, pad;
+  float hi, q_few, q_many, z_few, z_many, n_few, n_many;
   double z;
 };
 struct TaskLds {
@@ -355,12 +355,15 @@ static_assert(kSelQueue >= kThreads / kWaves * 8, "a quad step of a wave fits th
 // last stats work-group of the row; fused mode in every work-group of the row
 // once all slices have published (each computes the same result).
 //
-// One wave does the work with wave-level scans (no work-group barriers): one
-// round trip fetches the slice headers and the top 256 bins of every slice,
-// which are aligned through LDS; the bins are scanned from the top in blocks
-// of 64 and the scan stops at the block holding the cut.  Deeper cuts read
-// further bins, already aligned, 256 at a time.  Slices publish their own
-// total mass, so the scan never needs the bins below the cut.
+// One round trip fetches the slice headers and the top 256 or 512 bins of every
+// slice, which are aligned through LDS and scanned from the top; the scan stops
+// at the cut.  Deeper cuts read further bins, already aligned, 256 at a time.
+// Slices publish their own total mass, so the scan never needs the bins below
+// the cut.  The fused kernel (merge_stage, then merge_bins<true>) spreads the
+// round trip and the scan of those bins over the whole work-group, all of whose
+// threads enter both (they hold barriers), wave 0 the rest; split mode
+// (merge_bins<false>) is one wave with wave-level scans and no barrier.
+
 // The merge's first round trip, spread over the work-group: every wave reads
 // the slices' top bins and counts, wave 0 the rest of the heads (kept in LDS
 // for merge_bins), and wave s < G the top bins of slice s, which it adds,
@@ -2206,37 +2209,37 @@ __device__ __forceinline__ bool short_fallback(const Workspace& ws, int row, int
 // work-group, the counts complete.
 __device__ __forceinline__ int find_count_bin(TaskLds& L, uint32_t need) {
   const int tid = fresh_tid();
-            if (tid < 64) {
-              constexpr int kPer = kTauBins / 64;
-              uint32_t cb[kPer];
-              uint32_t cs = 0u;
-  #pragma unroll
-              for (int i = 0; i < kPer; ++i) {
-                cb[i] = L.sh.tcnt[kPer * tid + i];
-                cs += cb[i];
-              }
-              const uint32_t ic = wave_incl_scan(cs);
-              const uint64_t hit = __ballot(ic >= need);
-              int bs = kTauBins;  // the counts never reach `need`
-              if (hit) {
-                // first bin of each lane's run where the running count reaches
-                // k; lane f's is the answer
-                uint32_t acc = ic - cs;
-                int pos = kPer - 1;
-                bool found = false;
-  #pragma unroll
-                for (int i = 0; i < kPer; ++i) {
-                  acc += cb[i];
-                  const bool h = !found && acc >= need;
-                  pos = h ? i : pos;
-                  found = found || h;
-                }
-                const int f = __builtin_ctzll(hit);
-                bs = kPer * f + read_lane(pos, f);
-              }
-              if (tid == 0) L.misc[6] = bs;
-            }
-            __syncthreads();
+  if (tid < 64) {
+    constexpr int kPer = kTauBins / 64;
+    uint32_t cb[kPer];
+    uint32_t cs = 0u;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      cb[i] = L.sh.tcnt[kPer * tid + i];
+      cs += cb[i];
+    }
+    const uint32_t ic = wave_incl_scan(cs);
+    const uint64_t hit = __ballot(ic >= need);
+    int bs = kTauBins;  // the counts never reach `need`
+    if (hit) {
+      // first bin of each lane's run where the running count reaches
+      // k; lane f's is the answer
+      uint32_t acc = ic - cs;
+      int pos = kPer - 1;
+      bool found = false;
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) {
+        acc += cb[i];
+        const bool h = !found && acc >= need;
+        pos = h ? i : pos;
+        found = found || h;
+      }
+      const int f = __builtin_ctzll(hit);
+      bs = kPer * f + read_lane(pos, f);
+    }
+    if (tid == 0) L.misc[6] = bs;
+  }
+  __syncthreads();
   return L.misc[6];
 }
 
@@ -2654,14 +2657,15 @@ __device__ __forceinline__ bool nucleus_row(const Workspace& ws, const SamplePla
   int nq = 0;
 #pragma unroll
   for (int i = 0; i < kNucPer; ++i) {
-    if (i >= slots) break;
-    const float x = __uint_as_float((uint32_t)(kv[i] >> 32));
-    const bool in = pos + i * tp < my_n && row_top - bin_of(x, c.c32) <= info.cut;
-    const uint64_t b = __ballot(in);
-    if (in)
-      q[nq + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32),
-                                            __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0u))] = kv[i];
-    nq += (int)__popcll(b);
+    if (i < slots) {
+      const float x = __uint_as_float((uint32_t)(kv[i] >> 32));
+      const bool in = pos + i * tp < my_n && row_top - bin_of(x, c.c32) <= info.cut;
+      const uint64_t b = __ballot(in);
+      if (in)
+        q[nq + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32),
+                                              __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0u))] = kv[i];
+      nq += (int)__popcll(b);
+    }
   }
   __builtin_amdgcn_wave_barrier();
   double ent = 0.0;
