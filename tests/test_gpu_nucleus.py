@@ -10,6 +10,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
+import oracle as O
 from common import compare, rows_from_lists, run_gpu, run_oracle, to_torch_logits
 from lsamp import _ffi
 from lsamp import workloads as W
@@ -263,3 +264,15 @@ def test_ties_in_the_cut_bin(ctx, n):
     g = run_gpu(ctx, cfg)
     assert rows_from_lists(ctx, rows).all()
     compare(cfg, g, o, label=f"{n} ties")
+
+
+def test_keyed_draw_from_lists(ctx):
+    """Philox keys: a row's uniform is its key's, drawn by the row's last arriver."""
+    rows = 64
+    cfg = _batch(rows, 65536, _ffi.DTYPE_BF16, _ffi.SEM_CBV2, 5, False)
+    keys = np.array([O.rng_key(77, 1000 + r, 3) for r in range(rows)], np.uint64)
+    u = np.array([O.rng_uniform(int(k), 0) for k in keys], np.float32)
+    g = run_gpu(ctx, cfg, philox_keys=keys)
+    top_p = np.array([p["top_p"] < 1 for p in cfg["params"]])
+    assert rows_from_lists(ctx, rows)[top_p].any()
+    compare(cfg, g, run_oracle(cfg, philox_keys=keys, threads=16), label="keys", uniforms=u)
